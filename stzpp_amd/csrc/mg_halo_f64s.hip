@@ -1,0 +1,6 @@
+// Instances of the one-launch sweep (mg_instances.hpp).
+#include "mg_instances.hpp"
+
+namespace stzmg {
+STZ_HALO_SYM(, double)
+}  // namespace stzmg

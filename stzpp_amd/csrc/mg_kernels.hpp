@@ -512,7 +512,7 @@ __global__ void k_rat(Dims F, Dims C, const double *__restrict__ opsF, double *_
 // workgroup; ncls tables of kBlk values.
 constexpr int kSymThreads = 1024;
 constexpr double kCentroTol = 1e-13;  // rtol of k_centro_sym as the library uses it
-__global__ __launch_bounds__(kSymThreads) void k_centro_sym(double *__restrict__ ops, long ncls, double rtol) {
+static __global__ __launch_bounds__(kSymThreads) void k_centro_sym(double *__restrict__ ops, long ncls, double rtol) {
     __shared__ double red[kSymThreads / 64];
     const long ne = ncls * kBlk, np = ncls * 117;  // 13 blocks x 9 entries per plane
     double m = 0;
@@ -547,7 +547,7 @@ __global__ __launch_bounds__(kSymThreads) void k_centro_sym(double *__restrict__
 // counting as nonzero), out[27] = 1 when block(o) equals block(-o) bit for
 // bit in every plane.  One workgroup of kThreads.
 constexpr int kCfgWords = 28;
-__global__ __launch_bounds__(kThreads) void k_level_config(const double *__restrict__ ops, long ncls,
+static __global__ __launch_bounds__(kThreads) void k_level_config(const double *__restrict__ ops, long ncls,
                                                            unsigned *__restrict__ out) {
     __shared__ unsigned used[27];
     if (threadIdx.x < 27) used[threadIdx.x] = 0;
@@ -571,7 +571,7 @@ __global__ __launch_bounds__(kThreads) void k_level_config(const double *__restr
 // Centre-block inverse by cofactors over the determinant (src/mat3.hh:177-183)
 // and FP32 copies of the table.  flag[0] is set when a determinant is zero
 // or not finite.
-__global__ void k_inverse(const double *__restrict__ ops, long ncls, double *__restrict__ inv64,
+static __global__ void k_inverse(const double *__restrict__ ops, long ncls, double *__restrict__ inv64,
                           float *__restrict__ inv32, int *__restrict__ flag) {
     const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= ncls) return;
@@ -594,13 +594,13 @@ __global__ void k_inverse(const double *__restrict__ ops, long ncls, double *__r
     }
 }
 
-__global__ void k_cast_d2f(const double *__restrict__ a, float *__restrict__ b, long n) {
+static __global__ void k_cast_d2f(const double *__restrict__ a, float *__restrict__ b, long n) {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t < n) b[t] = (float)a[t];
 }
 
 // Deterministic final reduction of per-block partial pairs.
-__global__ void k_reduce_partials(const double *__restrict__ part, long nb, double *__restrict__ out) {
+static __global__ void k_reduce_partials(const double *__restrict__ part, long nb, double *__restrict__ out) {
     __shared__ double sa[1024], sb[1024];
     double a = 0, b = 0;
     for (long q = threadIdx.x; q < nb; q += blockDim.x) {
@@ -624,14 +624,14 @@ __global__ void k_reduce_partials(const double *__restrict__ part, long nb, doub
 }
 
 // AoS (3 per point) <-> SoA (component-major).
-__global__ void k_aos_to_soa(const double *__restrict__ a, double *__restrict__ s, long N) {
+static __global__ void k_aos_to_soa(const double *__restrict__ a, double *__restrict__ s, long N) {
     const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= N) return;
     s[p] = a[3 * p];
     s[p + N] = a[3 * p + 1];
     s[p + 2 * N] = a[3 * p + 2];
 }
-__global__ void k_soa_to_aos(const double *__restrict__ s, double *__restrict__ a, long N) {
+static __global__ void k_soa_to_aos(const double *__restrict__ s, double *__restrict__ a, long N) {
     const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= N) return;
     a[3 * p] = s[p];
@@ -669,7 +669,7 @@ __global__ __launch_bounds__(kThreads) void k_defect_f32(const TI *__restrict__ 
 }
 
 // x64 += s * e32.
-__global__ void k_update_f64(double *__restrict__ x, const float *__restrict__ e, double s, long n) {
+static __global__ void k_update_f64(double *__restrict__ x, const float *__restrict__ e, double s, long n) {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t < n) x[t] += s * (double)e[t];
 }

@@ -1,0 +1,6 @@
+// Instances of the marching residual kernel (mg_instances.hpp).
+#include "mg_instances.hpp"
+
+namespace stzmg {
+STZ_RESID_ALL(, double)
+}  // namespace stzmg

@@ -24,6 +24,7 @@
 #include "mg_kernels.hpp"
 #include "mg_march.hpp"
 #include "mg_resid.hpp"
+#include "mg_instances.hpp"
 #include "mg_krylov.hpp"
 
 using namespace stzmg;
@@ -221,19 +222,6 @@ double *pkr_of<double>(Level &L) { return L.pkr64; }
 template <>
 float *pkr_of<float>(Level &L) { return L.pkr32; }
 
-// Tiles of the plane-marching residual (k_resid_march): 64 x 16 in FP32,
-// 32 x 16 in FP64, 256 threads.
-template <typename T>
-struct ResidTile;
-template <>
-struct ResidTile<float> {
-    static constexpr int TX = 64, TY = 16;
-};
-template <>
-struct ResidTile<double> {
-    static constexpr int TX = 32, TY = 16;
-};
-
 bool tiled_ok(const Level &L) {
     return L.mode == STZMG_OP_PLANE && L.d.px && L.d.py && L.d.m % ResidTile<float>::TX == 0 &&
            L.d.n % ResidTile<float>::TY == 0 && L.d.m % ResidTile<double>::TX == 0 &&
@@ -244,7 +232,6 @@ bool tiled_ok(const Level &L) {
 // plane levels periodic in x and y that the tiles above do not divide (the
 // 96^2 and 48^2 levels of a 192^2 grid, 32^3 and 16^3 below 256^3); used for
 // the V-cycle's residuals, which take no norm partials.
-constexpr int kResidSmall = 16;
 bool tiled_small_ok(const Level &L) {
     return L.mode == STZMG_OP_PLANE && L.d.px && L.d.py && !tiled_ok(L) && L.d.m % kResidSmall == 0 &&
            L.d.n % kResidSmall == 0;
@@ -384,42 +371,6 @@ void launch_apply(stzmg_t h, Level &L, const T *x, T *out, T *xcopy = nullptr) {
 
 int ncol(int n, int prd) { return (prd && (n & 1)) ? 3 : 2; }
 
-// Tile and workgroup size of the large fused-smoother class (k_gs_march):
-// 64 x 16 with 512 threads in FP32 (three staged planes of 71 x 24 points,
-// 61,344 B of LDS: two workgroups per CU) and 32 x 16 with 256 threads in
-// FP64 (39 x 24 points, 67,392 B: two per CU).  Measured on the 256^3
-// transformed-operator sweep (MI355X): FP32 64 x 16 / 512 threads 0.256 ms,
-// 64 x 8 / 256 0.272 ms, 32 x 16 / 256 0.291 ms; FP64 32 x 16 0.519 ms,
-// 32 x 8 0.666 ms.
-#ifndef STZ_F32_TX
-#define STZ_F32_TX 64
-#endif
-#ifndef STZ_F32_TY
-#define STZ_F32_TY 16
-#endif
-#ifndef STZ_F32_NT
-#define STZ_F32_NT 512
-#endif
-#ifndef STZ_F64_TX
-#define STZ_F64_TX 32
-#endif
-#ifndef STZ_F64_TY
-#define STZ_F64_TY 16
-#endif
-#ifndef STZ_F64_NT
-#define STZ_F64_NT 256
-#endif
-template <typename T>
-struct FusedTile;
-template <>
-struct FusedTile<float> {
-    static constexpr int TX = STZ_F32_TX, TY = STZ_F32_TY, NT = STZ_F32_NT;
-};
-template <>
-struct FusedTile<double> {
-    static constexpr int TX = STZ_F64_TX, TY = STZ_F64_TY, NT = STZ_F64_NT;
-};
-
 template <typename T>
 T *&xb_of(Level &L);
 template <>
@@ -437,42 +388,44 @@ float *&xref_of<float>(Level &L) { return L.x32; }
 // tiles with 128 threads: one thread per point of the widest sub-pass.
 // Sides that are multiples of 8 only (e.g. 24 x 24, a level of the
 // 192 x 192 grids) use 8 x 8 tiles with one wave.
-constexpr int kSmallTile = 16, kSmallThreads = 128;
-constexpr int kTinyTile = 8, kTinyThreads = 64;
-
-// Fused-smoother tile class of a level for sweeps in type T: 0 none, 1 the
-// large tiles of T (64 x 8 FP32, 32 x 16 FP64), 2 the 16 x 16 tiles, 3 the
-// 8 x 8 tiles.  The largest tile that divides the
-// plane is taken unless one launch would then have fewer than
-// STZ_FUSED_MIN_GROUPS workgroups (tiles times planes of one parity) and a
-// smaller tile divides the plane too.
-#ifndef STZ_FUSED_MIN_GROUPS
-#define STZ_FUSED_MIN_GROUPS 0
-#endif
-template <typename T>
-int fused_tile(const Level &L) {
-    if (!(L.mode == STZMG_OP_PLANE && L.d.px && L.d.py && L.d.o >= 4 && L.d.N > 1024)) return 0;
-    const long nP = (L.d.o + 1) / 2;
-    auto groups = [&](int tx, int ty) { return (long)(L.d.m / tx) * (L.d.n / ty) * nP; };
-    int best = 0;
-    if (L.d.m % FusedTile<T>::TX == 0 && L.d.n % FusedTile<T>::TY == 0) {
-        best = 1;
-        if (groups(FusedTile<T>::TX, FusedTile<T>::TY) >= STZ_FUSED_MIN_GROUPS) return best;
-    }
-    if (L.d.m % kSmallTile == 0 && L.d.n % kSmallTile == 0) {
-        best = 2;
-        if (groups(kSmallTile, kSmallTile) >= STZ_FUSED_MIN_GROUPS) return best;
-    }
-    if (L.d.m % kTinyTile == 0 && L.d.n % kTinyTile == 0) best = 3;
-    return best;
-}
-
-// Every tile class sweeps with the z-marching kernel k_gs_march
+// Tile classes 1 to 3 sweep with the z-marching kernel k_gs_march
 // (mg_march.hpp); STZ_MARCH=0 builds the staged-broadcast one-plane kernel
 // k_gs_planes instead (for comparison; without the zero-start sweeps).
 #ifndef STZ_MARCH
 #define STZ_MARCH 1
 #endif
+
+// The one-launch sweep k_gs_halo takes a level whose tiles (8 x 8 points of a
+// plane pair) fill the chip at most twice over: 512 workgroups, two on each
+// of the 256 CUs (a fixed number, so that the smoother's rounding does not
+// depend on the device).  Up to there the sweep is a chain of latencies and
+// one launch beats two; beyond, its recomputed halo costs more than the
+// launch (us per sweep, marching against one launch: 48 x 40 x 25, 390
+// workgroups, dense FP64 19.8 / 15.8, FP32 16.7 / 13.4; 48 x 48 x 24, 432,
+// shear FP64 14.4 / 13.1; 48 x 48 x 49, 900, FP64 15.0 / 21.0, FP32
+// 11.8 / 14.5; 64 x 64 x 33, 1088, FP64 18.4 / 30.5).  It also takes every
+// level that no marching tile divides, whose alternative is eight colour
+// launches (24 x 20 x 13 FP64 51 / 11.0).
+constexpr long kHaloGroups = 512;
+
+// Fused-smoother tile class of a level for sweeps in type T: 0 none, 1 the
+// large marching tiles of T (64 x 16 FP32, 32 x 16 FP64), 2 the 16 x 16
+// tiles, 3 the 8 x 8 tiles (the largest that divides the plane), 4 the
+// one-launch sweep.
+template <typename T>
+int fused_tile(const Level &L) {
+    const Dims &d = L.d;
+    if (!(L.mode == STZMG_OP_PLANE && d.px && d.py && d.o >= 4 && d.N > 1024)) return 0;
+    int best = 0;
+    if (d.m % FusedTile<T>::TX == 0 && d.n % FusedTile<T>::TY == 0) best = 1;
+    else if (d.m % kSmallTile == 0 && d.n % kSmallTile == 0) best = 2;
+    else if (d.m % kTinyTile == 0 && d.n % kTinyTile == 0) best = 3;
+    const bool halo = STZ_MARCH != 0 && d.m % 2 == 0 && d.n % 2 == 0 && d.m >= 8 && d.n >= 8 && (!d.pz || d.o % 2 == 0);
+    const long groups = (long)((d.m + kHaloTile - 1) / kHaloTile) * ((d.n + kHaloTile - 1) / kHaloTile) * ((d.o + 1) / 2);
+    if (halo && (best == 0 || groups <= kHaloGroups)) return 4;
+    return best;
+}
+
 template <typename T, int PAT, int TX, int TY, int NT, bool MARCH>
 const void *sweep_kernel() {
     if constexpr (MARCH)
@@ -543,9 +496,32 @@ void launch_fused_tile(stzmg_t h, Level &L, bool zero_start = false) {
     std::swap(xref_of<T>(L), xb_of<T>(L));
 }
 
+// One sweep in one launch (mg_halo.hpp).
+template <typename T, int KEY>
+void launch_halo(stzmg_t h, Level &L, bool zero_start) {
+    const Dims &d = L.d;
+    constexpr int TX = kHaloTile;
+    T *x = xref_of<T>(L), *xb = xb_of<T>(L);
+    const dim3 g((d.m + TX - 1) / TX, (d.n + TX - 1) / TX, (d.o + 1) / 2);
+    const bool rec = h->launch_ev && h->launch_ev_next + 2 <= h->launch_ev->size();
+    if (rec) (void)hipEventRecord((*h->launch_ev)[h->launch_ev_next], h->stream);
+    hipLaunchKernelGGL((k_gs_halo<T, KEY, TX, TX>), g, dim3(halo_threads<TX, TX>()), 0, h->stream, d, (const T *)x, xb,
+                       (const T *)r_of<T>(L), (const T *)pk_of<T>(L), zero_start ? 1 : 0);
+    if (rec) {
+        (void)hipEventRecord((*h->launch_ev)[h->launch_ev_next + 1], h->stream);
+        h->launch_ev_next += 2;
+    }
+    std::swap(xref_of<T>(L), xb_of<T>(L));
+}
+
 template <typename T, int PAT>
 void launch_fused_pat(stzmg_t h, Level &L, bool zero_start) {
     const int ft = sizeof(T) == 4 ? L.ftile : L.ftile64;
+    if (ft == 4) {
+        if (L.sym) launch_halo<T, PAT + kMarchSym>(h, L, zero_start);
+        else launch_halo<T, PAT>(h, L, zero_start);
+        return;
+    }
     if (ft == 1) {
         constexpr int TX = FusedTile<T>::TX, TY = FusedTile<T>::TY, NT = FusedTile<T>::NT;
         if constexpr (STZ_MARCH != 0) {
@@ -586,8 +562,8 @@ void launch_gs_sweep_colours(stzmg_t h, Level &L);
 // memory (the fused sweep k_gs_march skips the planes it knows are zero).
 bool zero_start_ok(const Level &L) { return STZ_MARCH != 0 && L.fused; }
 
-// One Gauss-Seidel sweep of a level: two fused launches where the level
-// allows, eight colour launches otherwise.  zero_start (only where
+// One Gauss-Seidel sweep of a level: one or two fused launches where the
+// level allows, eight colour launches otherwise.  zero_start (only where
 // zero_start_ok): the sweep starts from x = 0 whatever x holds.
 template <typename T>
 void launch_gs_sweep(stzmg_t h, Level &L, bool zero_start = false) {

@@ -1,0 +1,103 @@
+"""The one-launch sweep (k_gs_halo) against the oracle's 8-colour sweep.
+
+Sizes where it can go wrong: the smallest planes (8, 10 and 12 points wide:
+the 24-point window wraps up to three times), tiles that stick out of the
+plane (sides not multiples of 8), the fewest planes, an even number of
+periodic planes against an odd number between walls, the largest level it
+takes while a marching tile divides the plane (512 workgroups) and the first
+one beyond, and sides that only it sweeps fused.  Each zero pattern, plain
+and centrosymmetric.
+
+Bounds: a sweep forms each value from 27 x 9 products, so FP64 rounding
+stays below a few hundred ulp of the largest value over three sweeps
+(1e-12), and FP32 below 2e-6 for one sweep on FP32-rounded inputs.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+from stzpp_amd import multigrid as MG
+
+pytestmark = pytest.mark.gpu
+
+T_XZ = np.array([[1.0, 0.0, 0.5], [0.0, 1.0, 0.0], [0.0, 0.0, 1.0]])
+T_FULL = np.array([[1.1, 0.2, 0.3], [0.0, 0.9, 0.1], [0.0, 0.0, 1.0]])
+
+
+def relerr(a, b):
+    return float(np.abs(a - b).max() / np.abs(b).max())
+
+
+def f32(a):
+    return np.asarray(a, dtype=np.float32).astype(np.float64)
+
+
+def planes_of(kind, m, n, o, pz):
+    hx, hy, hz = 1.0 / m, 1.0 / n, 1.0 / o
+    st, fix = MG.shear_stencil(1.0, 1.5, hx, hy, hz, 1.0)
+    if kind in ("trans", "full"):
+        st = MG.trans_stencil(T_XZ if kind == "trans" else T_FULL, 1.0, 1.5, hx, hy, hz, 1.0)
+    elif kind == "dense":
+        # centrosymmetric dense blocks: a Galerkin level of a periodic problem
+        big = MG.Multigrid(64, 64, 64, (1, 1, 1))
+        big.setup_matrices_const(MG.trans_stencil(T_XZ, 1.0, 1.5, hx, hy, hz, 1.0), None)
+        st = big.level_operator(1)[0]
+    planes = O.plane_operator(o, pz, st, None if pz else fix)
+    if kind == "plain":
+        # not centrosymmetric: a perturbed dense stencil, another one per plane
+        rng = np.random.default_rng(5)
+        planes = np.array(planes).reshape(o, 27, 3, 3)
+        planes += 0.02 * np.abs(planes).max() * rng.uniform(-1, 1, planes.shape) * (planes.any(axis=(1, 2, 3)))[
+            :, None, None, None]
+        if not pz:
+            planes[0, :9] = 0
+            planes[-1, 18:] = 0
+    return np.ascontiguousarray(planes)
+
+
+SIZES = [(8, 16, 16, 1), (10, 14, 9, 0), (12, 12, 13, 0), (12, 10, 10, 1), (16, 20, 4, 1), (20, 28, 5, 0),
+         (18, 22, 13, 0), (32, 24, 16, 1), (64, 64, 16, 1), (64, 64, 17, 0), (36, 44, 25, 0), (72, 72, 17, 0)]
+
+
+@pytest.mark.parametrize("m,n,o,pz", SIZES)
+@pytest.mark.parametrize("kind", ["shear", "trans", "full", "dense", "plain"])
+def test_one_launch_sweep(kind, m, n, o, pz):
+    prd = (1, 1, pz)
+    planes = planes_of(kind, m, n, o, pz)
+    N = m * n * o
+    x, r = O.det_field(N, 11), O.det_field(N, 12)
+    mg = MG.Multigrid(m, n, o, prd, coarsest_total=N)  # this level alone
+    mg.setup_matrices_planes(planes)
+    orc = O.OracleMG(m, n, o, prd, mode=O.PLANE, coarsest_total=N)
+    orc.set_ops(0, planes)
+    orc.params(smoother=1)
+    mg.setup_fields(x, r)
+    orc.set_fields(0, x, r)
+    mg.gauss_seidel(0, 3)
+    orc.gs(0, 3)
+    assert relerr(mg.x(0), orc.fields(0)[0]) < 1e-12
+    mg.setup_fields(x, r)
+    orc.set_fields(0, f32(x), f32(r))
+    mg.gauss_seidel_fp32(0, 1)
+    orc.gs(0, 1)
+    assert relerr(mg.x(0), orc.fields(0)[0]) < 2e-6
+
+
+@pytest.mark.parametrize("m,n,o,pz", [(20, 28, 17, 0), (24, 32, 16, 1), (16, 16, 17, 0)])
+def test_vcycle_from_zero(m, n, o, pz):
+    """V-cycles through one-launch levels, whose first sweep starts from
+    x = 0 without reading it, against the oracle's."""
+    prd = (1, 1, pz)
+    st, fix = MG.shear_stencil(1.0, 1.5, 1.0 / m, 1.0 / n, 1.0 / o, 1.0)
+    mg = MG.Multigrid(m, n, o, prd)
+    mg.setup_matrices_const(st, None if pz else fix)
+    orc = O.OracleMG(m, n, o, prd, mode=O.PLANE)
+    orc.set_ops(0, O.plane_operator(o, pz, st, None if pz else fix))
+    orc.rat()
+    orc.params(smoother=1)
+    x, r = O.det_field(m * n * o, 21), O.det_field(m * n * o, 22)
+    mg.setup_fields(x, r)
+    orc.set_fields(0, x, r)
+    mg.v_cycle(2)
+    orc.vcycle(2)
+    assert relerr(mg.x(0), orc.fields(0)[0]) < 1e-11
