@@ -300,7 +300,7 @@ int stz_create(const stz_params *p, stz_t *out) {
     A(&s->vel, 3 * Nv); A(&s->sig, 6 * Nc); A(&s->sig2, 6 * Nc); A(&s->chi, Nc); A(&s->chi2, Nc);
     A(&s->dpl, Nc); A(&s->dpl2, Nc); A(&s->adapt, Nc); A(&s->dchi, Nc);
     A(&s->stage, 6 * (Nc > Nv ? Nc : Nv));
-    if (e == hipSuccess) e = hipMalloc((void **)&s->counters, sizeof(int) * 4);
+    if (e == hipSuccess) e = hipMalloc((void **)&s->counters, sizeof(int) * kCountInts);
     A(&s->pm_part, (long)nb(Nc) + 1);
     if (e != hipSuccess) {
         g_stz_err = "device allocation failed";
@@ -439,7 +439,7 @@ int step_once(stz_t s, double dt, stzmg_solve_opts &o, bool ref_tol, stz_step_st
     const bool trans = s->p.transform != STZ_T_NONE;
     const Grid &g = s->g;
     const Box box{s->p.ax, s->p.ay, s->p.az, s->p.bx, s->p.by, s->p.bz};
-    SHIP(s, hipMemsetAsync(s->counters, 0, sizeof(int) * 4, s->stream));
+    SHIP(s, hipMemsetAsync(s->counters, 0, sizeof(int) * kCountInts, s->stream));
     if (trans) {
         const Xform Xn = xform_at(s, s->t);
         hipLaunchKernelGGL(k_plastic_trans, dim3(nb(g.Nc)), dim3(kT), 0, s->stream, g, s->M, dt, Xn,
@@ -494,13 +494,13 @@ int step_once(stz_t s, double dt, stzmg_solve_opts &o, bool ref_tol, stz_step_st
                            s->pm_part + nb(g.Nc));
     }
     SHIP(s, hipGetLastError());
-    int cnt[4];
+    int cnt[kCountInts];
     double pm = 0;
     SHIP(s, hipMemcpyAsync(cnt, s->counters, sizeof(cnt), hipMemcpyDeviceToHost, s->stream));
     if (!trans) SHIP(s, hipMemcpyAsync(&pm, s->pm_part + nb(g.Nc), sizeof(double), hipMemcpyDeviceToHost, s->stream));
     SHIP(s, hipStreamSynchronize(s->stream));
     s->proj_mag = pm;
-    S.yielded_cells = cnt[0];
+    S.yielded_cells = count_total(cnt);
     S.steps++;
     return step_output(s);
 }

@@ -97,7 +97,7 @@ static __global__ __launch_bounds__(kT) void k_direct_plastic(Grid g, Mat M, dou
         a = adaptive(M, sb, chi[c], dt, dc, n);
         D = a / 2. / M.mu / dt * sb;
     }
-    count_wave(&counters[0], sb > M.sy);
+    count_wave(counters, sb > M.sy);
     adapt[c] = a;
     dchi[c] = dc;
     dpl_new[c] = D;
@@ -471,7 +471,7 @@ int stz_step_direct(stz_t s, double dt, int nsteps, stz_step_stats *st) {
     const BrickGrid bc = brick_grid(g.Nx, g.Ny, g.Nz), bv = brick_grid(g.Nx, g.Ny, g.Nzv);
     stz_step_stats S{};
     for (int q = 0; q < nsteps; q++) {
-        DHIP(s, hipMemsetAsync(s->counters, 0, sizeof(int) * 4, s->stream));
+        DHIP(s, hipMemsetAsync(s->counters, 0, sizeof(int) * kCountInts, s->stream));
         hipLaunchKernelGGL(k_direct_plastic, dim3(nbk(g.Nc)), dim3(kT), 0, s->stream, g, s->M, dt,
                            (const double *)s->sig, (const double *)s->chi, s->adapt, s->dchi, s->dpl2, s->counters);
         hipLaunchKernelGGL(k_direct_cell, dim3(brick_blocks(bc)), dim3(kT), 0, s->stream, g, s->M, dt,
@@ -494,10 +494,10 @@ int stz_step_direct(stz_t s, double dt, int nsteps, stz_step_stats *st) {
         S.steps++;
     }
     // one synchronisation per call: the counters hold the last step's count
-    int cnt[4] = {0, 0, 0, 0};
+    int cnt[kCountInts];
     DHIP(s, hipMemcpyAsync(cnt, s->counters, sizeof(cnt), hipMemcpyDeviceToHost, s->stream));
     DHIP(s, hipStreamSynchronize(s->stream));
-    S.yielded_cells = nsteps ? cnt[0] : 0;
+    S.yielded_cells = nsteps ? count_total(cnt) : 0;
     if (st) *st = S;
     return 0;
 }
