@@ -119,6 +119,87 @@ __device__ __forceinline__ float row16_sum(float v) {
 // a point differs.  On exit x holds the result.
 constexpr int kBottomLanes = 16;
 static_assert(kBottomLanes == 16, "row16_sum reduces rows of 16 lanes");
+// The same sweeps of a per-plane level whose colours have at most one point
+// per group of lanes (x and y periodic and even, 8 x 8 x 8 and smaller in a
+// workgroup of 1024): a lane keeps its plane pair's blocks, its inverse row
+// and its neighbours' index parts in registers through all sweeps, so a pass
+// is six LDS reads, the multiply-adds, the lane sums and one write (lanes 0 to
+// 2 write one component each).  Computing indices and re-reading the tables
+// in every pass had kept the SIMDs busy longer than the arithmetic: 24 sweeps
+// of 8 x 8 x 4 points took 265 us, 1.4 us a pass (100 us, 0.5 us here).
+__host__ __device__ inline bool bottom_in_registers(const Dims &d) {
+    return d.px && d.py && !(d.m & 1) && !(d.n & 1) && !(d.pz && (d.o & 1)) &&
+           (d.m / 2) * (d.n / 2) * ((d.o + 1) / 2) <= kCoarseThreads / kBottomLanes;
+}
+template <typename T>
+__device__ void wg_bottom_sweeps_reg(const Dims &d, const T *ops, const T *inv, int nsweeps, T *xs, const T *rs) {
+    const int N = (int)d.N;
+    const int sl = threadIdx.x % kBottomLanes, grp = threadIdx.x / kBottomLanes;
+    const int cntx = d.m / 2, cnty = d.n / 2, tot = cntx * cnty * ((d.o + 1) / 2);
+    const int g = grp < tot ? grp : 0;
+    const int ii = g % cntx, rest = g / cntx, jj = rest % cnty, kk = rest / cnty;
+    // blocks h = 0, 1 of this lane, by plane parity; index parts of the
+    // neighbour by colour.  A block that does not exist (the centre, beyond
+    // the list, across a wall) is zero and reads the point itself.
+    T A[2][2][9], B[2][3];
+    int qx[2][2], qy[2][2], qz[2][2], pz[2];
+    bool own[2];
+#pragma unroll
+    for (int cz = 0; cz < 2; cz++) {
+        const int k = cz + 2 * kk, kc = k < d.o ? k : 0;
+        own[cz] = grp < tot && k < d.o;
+        pz[cz] = 2 * ii + d.m * (2 * jj + d.n * kc);
+        const int row = sl < 3 ? sl : 0;
+#pragma unroll
+        for (int e = 0; e < 3; e++) B[cz][e] = inv[kc * 9 + 3 * row + e];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int b = sl + kBottomLanes * h;
+            const int nk = b < 27 ? nb(kc, b / 9 - 1, d.o, d.pz) : -1;
+            const bool ok = b < 27 && b != 13 && nk >= 0;
+            qz[h][cz] = d.m * d.n * (ok ? nk : kc);
+#pragma unroll
+            for (int e = 0; e < 9; e++) A[cz][h][e] = ok ? ops[(long)kc * kBlk + 9 * b + e] : T(0);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int b = sl + kBottomLanes * h < 27 ? sl + kBottomLanes * h : 13;
+            qx[h][c] = nb(c + 2 * ii, b % 3 - 1, d.m, 1);
+            qy[h][c] = d.m * nb(c + 2 * jj, (b / 3) % 3 - 1, d.n, 1);
+        }
+    // the two neighbours' indices of each colour in one register
+    unsigned qq[8];
+#pragma unroll
+    for (int col = 0; col < 8; col++) {
+        const int cx = col & 1, cy = (col >> 1) & 1, cz = col >> 2;
+        qq[col] = (unsigned)(qx[0][cx] + qy[0][cy] + qz[0][cz]) |
+                  (unsigned)(qx[1][cx] + qy[1][cy] + qz[1][cz]) << 16;
+    }
+    // waves without a point only meet the barriers
+    const bool idle = (int)(threadIdx.x / 64) * (64 / kBottomLanes) >= tot;
+    for (int sw = 0; sw < nsweeps; sw++) {
+#pragma unroll
+        for (int col = 0; col < 8; col++) {
+            const int cx = col & 1, cy = (col >> 1) & 1, cz = col >> 2;
+            if (!idle) {
+                // unpacked here, not held unpacked through the sweeps
+                asm volatile("" : "+v"(qq[col]), "+v"(pz[cz]));
+                const int p = pz[cz] + cx + d.m * cy, q0 = (int)(qq[col] & 0xFFFFu), q1 = (int)(qq[col] >> 16);
+                // the first lane's sum starts from -r
+                T a0 = sl ? T(0) : -rs[p], a1 = sl ? T(0) : -rs[p + N], a2 = sl ? T(0) : -rs[p + 2 * N];
+                mv(A[cz][0], xs[q0], xs[q0 + N], xs[q0 + 2 * N], a0, a1, a2);
+                mv(A[cz][1], xs[q1], xs[q1 + N], xs[q1 + 2 * N], a0, a1, a2);
+                const T e0 = -row16_sum(a0), e1 = -row16_sum(a1), e2 = -row16_sum(a2);
+                if (own[cz] && sl < 3) xs[p + sl * N] = B[cz][0] * e0 + B[cz][1] * e1 + B[cz][2] * e2;
+            }
+            __syncthreads();
+        }
+    }
+}
+
 template <typename T, int MODE>
 __device__ void wg_bottom_sweeps(const Dims &d, const T *ops, const T *inv, int nsweeps, T *xs, const T *rs) {
     const long N = d.N;
@@ -181,7 +262,10 @@ __device__ void wg_bottom_solve(const Dims &d, T *x, const T *r, const T *ops, c
         rs[q] = r[q];
     }
     __syncthreads();
-    wg_bottom_sweeps<T, MODE>(d, ops, inv, nsweeps, xs, rs);
+    if (MODE == 0 && bottom_in_registers(d))
+        wg_bottom_sweeps_reg<T>(d, ops, inv, nsweeps, xs, rs);
+    else
+        wg_bottom_sweeps<T, MODE>(d, ops, inv, nsweeps, xs, rs);
     for (int q = threadIdx.x; q < n3; q += blockDim.x) x[q] = xs[q];
     __syncthreads();
 }
@@ -193,8 +277,10 @@ __device__ void wg_bottom_solve(const Dims &d, T *x, const T *r, const T *ops, c
 // as wg_bottom_solve, and stores it at q[i 3N + j]; k_bottom_apply then
 // replaces the single-workgroup bottom solve of every V-cycle by a
 // matrix-vector product spread over the GPU.  Dynamic LDS: the staged
-// per-plane tables (MODE 0; table_vals doubles) and x, r of the level.
-template <int MODE>
+// per-plane tables (MODE 0; table_vals doubles) and x, r of the level.  REG:
+// the sweeps of bottom_in_registers levels (an instance of its own: their
+// registers leave one workgroup per CU, the others' two).
+template <int MODE, bool REG>
 __global__ __launch_bounds__(kCoarseThreads) void k_bottom_map(Dims d, const double *ops, const double *inv,
                                                                int nsweeps, int table_vals, double *q) {
     extern __shared__ double coarse_lds[];
@@ -208,7 +294,10 @@ __global__ __launch_bounds__(kCoarseThreads) void k_bottom_map(Dims d, const dou
         rs[t] = t == j ? 1.0 : 0.0;
     }
     __syncthreads();
-    wg_bottom_sweeps<double, MODE>(d, ops_s, inv_s, nsweeps, xs, rs);
+    if constexpr (REG)
+        wg_bottom_sweeps_reg<double>(d, ops_s, inv_s, nsweeps, xs, rs);
+    else
+        wg_bottom_sweeps<double, MODE>(d, ops_s, inv_s, nsweeps, xs, rs);
     for (int i = threadIdx.x; i < n3; i += blockDim.x) q[(long)i * n3 + j] = xs[i];
 }
 

@@ -26,6 +26,7 @@
 #include "mg_resid.hpp"
 #include "mg_instances.hpp"
 #include "mg_krylov.hpp"
+#include "mg_points.hpp"
 
 using namespace stzmg;
 
@@ -602,15 +603,15 @@ void launch_gs_sweep_colours(stzmg_t h, Level &L) {
                 const int cntx = col_count(d.m, cx, d.px), cnty = col_count(d.n, cy, d.py),
                           cntz = col_count(d.o, cz, d.pz);
                 if (cntx == 0 || cnty == 0 || cntz == 0) continue;
+                if (L.mode == STZMG_OP_POINT) {
+                    hipLaunchKernelGGL((k_gs_points<T>), dim3(nblk((long)cntx * cnty * kPointLanes), cntz),
+                                       dim3(kThreads), 0, h->stream, d, x_of<T>(L), (const T *)r_of<T>(L),
+                                       ops_of<T>(L), inv_of<T>(L), cx, cy, cz, cntx, cnty);
+                    continue;
+                }
                 dim3 g(nblk((long)cntx * cnty), cntz);
-                if (L.mode == STZMG_OP_PLANE)
-                    hipLaunchKernelGGL((k_gs<T, 0>), g, dim3(kThreads), 0, h->stream, d, x_of<T>(L),
-                                       (const T *)r_of<T>(L), ops_of<T>(L), inv_of<T>(L), cx, cy, cz,
-                                       cntx, cnty);
-                else
-                    hipLaunchKernelGGL((k_gs<T, 1>), g, dim3(kThreads), 0, h->stream, d, x_of<T>(L),
-                                       (const T *)r_of<T>(L), ops_of<T>(L), inv_of<T>(L), cx, cy, cz,
-                                       cntx, cnty);
+                hipLaunchKernelGGL((k_gs<T, 0>), g, dim3(kThreads), 0, h->stream, d, x_of<T>(L),
+                                   (const T *)r_of<T>(L), ops_of<T>(L), inv_of<T>(L), cx, cy, cz, cntx, cnty);
             }
 }
 
@@ -674,7 +675,8 @@ int coarse_kernel_attrs(stzmg_t h) {
         hipError_t e = hipSuccess;
         const void *fns[] = {(const void *)k_coarse_cycle<float, 0>, (const void *)k_coarse_cycle<float, 1>,
                              (const void *)k_coarse_cycle<double, 0>, (const void *)k_coarse_cycle<double, 1>,
-                             (const void *)k_bottom_map<0>, (const void *)k_bottom_map<1>};
+                             (const void *)k_bottom_map<0, false>, (const void *)k_bottom_map<0, true>,
+                             (const void *)k_bottom_map<1, false>};
         for (const void *f : fns) {
             const hipError_t e1 = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCoarseLdsMax);
             if (e1 != hipSuccess) e = e1;
@@ -923,11 +925,14 @@ int build_bottom_map(stzmg_t h) {
         h->qmap_n = n3;
     }
     const int tv = (int)(tab / sizeof(double));
-    if (plane)
-        hipLaunchKernelGGL(k_bottom_map<0>, dim3((unsigned)n3), dim3(kCoarseThreads), bytes, h->stream, B.d,
+    if (plane && bottom_in_registers(B.d))
+        hipLaunchKernelGGL((k_bottom_map<0, true>), dim3((unsigned)n3), dim3(kCoarseThreads), bytes, h->stream, B.d,
+                           (const double *)B.ops64, (const double *)B.inv64, h->desc.bottom_sweeps, tv, h->qmap);
+    else if (plane)
+        hipLaunchKernelGGL((k_bottom_map<0, false>), dim3((unsigned)n3), dim3(kCoarseThreads), bytes, h->stream, B.d,
                            (const double *)B.ops64, (const double *)B.inv64, h->desc.bottom_sweeps, tv, h->qmap);
     else
-        hipLaunchKernelGGL(k_bottom_map<1>, dim3((unsigned)n3), dim3(kCoarseThreads), bytes, h->stream, B.d,
+        hipLaunchKernelGGL((k_bottom_map<1, false>), dim3((unsigned)n3), dim3(kCoarseThreads), bytes, h->stream, B.d,
                            (const double *)B.ops64, (const double *)B.inv64, h->desc.bottom_sweeps, tv, h->qmap);
     LAUNCHCHK(h);
     h->qmap_ok = true;
