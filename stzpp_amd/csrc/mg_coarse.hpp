@@ -125,8 +125,9 @@ static_assert(kBottomLanes == 16, "row16_sum reduces rows of 16 lanes");
 // and its neighbours' index parts in registers through all sweeps, so a pass
 // is six LDS reads, the multiply-adds, the lane sums and one write (lanes 0 to
 // 2 write one component each).  Computing indices and re-reading the tables
-// in every pass had kept the SIMDs busy longer than the arithmetic: 24 sweeps
-// of 8 x 8 x 4 points took 265 us, 1.4 us a pass (100 us, 0.5 us here).
+// in every pass had kept the SIMDs busy longer than the arithmetic (1.4 us a
+// pass at 8 x 8 x 4, 0.5 us here): the map of 8 x 8 x 8 points takes 1.1 ms
+// instead of 2.2.
 __host__ __device__ inline bool bottom_in_registers(const Dims &d) {
     return d.px && d.py && !(d.m & 1) && !(d.n & 1) && !(d.pz && (d.o & 1)) &&
            (d.m / 2) * (d.n / 2) * ((d.o + 1) / 2) <= kCoarseThreads / kBottomLanes;
@@ -262,10 +263,7 @@ __device__ void wg_bottom_solve(const Dims &d, T *x, const T *r, const T *ops, c
         rs[q] = r[q];
     }
     __syncthreads();
-    if (MODE == 0 && bottom_in_registers(d))
-        wg_bottom_sweeps_reg<T>(d, ops, inv, nsweeps, xs, rs);
-    else
-        wg_bottom_sweeps<T, MODE>(d, ops, inv, nsweeps, xs, rs);
+    wg_bottom_sweeps<T, MODE>(d, ops, inv, nsweeps, xs, rs);
     for (int q = threadIdx.x; q < n3; q += blockDim.x) x[q] = xs[q];
     __syncthreads();
 }
