@@ -444,7 +444,7 @@ int stz_set_ref_map(stz_t s, const double *xi) {
     if (!s || !xi) return STZMG_ERR_ARG;
     if (int rc = ensure_ref_map(s)) return rc;
     const Grid &g = s->g;
-    DHIP(s, hipMemcpyAsync(s->stage, xi, sizeof(double) * 3 * g.Nv, hipMemcpyHostToDevice, s->stream));
+    DHIP(s, s->ring.upload(s->stage, xi, sizeof(double) * 3 * g.Nv, s->stream));
     hipLaunchKernelGGL(k_aos2soa, dim3(nbk(g.Nv)), dim3(kT), 0, s->stream, (const double *)s->stage, s->xi, g.Nv, 3);
     DHIP(s, hipGetLastError());
     DHIP(s, hipStreamSynchronize(s->stream));
@@ -457,8 +457,7 @@ int stz_get_ref_map(stz_t s, double *xi) {
     const Grid &g = s->g;
     hipLaunchKernelGGL(k_soa2aos, dim3(nbk(g.Nv)), dim3(kT), 0, s->stream, (const double *)s->xi, s->stage, g.Nv, 3);
     DHIP(s, hipGetLastError());
-    DHIP(s, hipMemcpyAsync(xi, s->stage, sizeof(double) * 3 * g.Nv, hipMemcpyDeviceToHost, s->stream));
-    DHIP(s, hipStreamSynchronize(s->stream));
+    DHIP(s, s->ring.download(xi, s->stage, sizeof(double) * 3 * g.Nv, s->stream));
     return 0;
 }
 

@@ -7,6 +7,7 @@
 #include <string>
 
 #include "../../include/stz.h"
+#include "host_copy.hpp"
 #include "stz_kernels.hpp"
 
 struct stz_s {
@@ -22,6 +23,7 @@ struct stz_s {
     double *vel = nullptr, *sig = nullptr, *sig2 = nullptr, *chi = nullptr, *chi2 = nullptr;
     double *dpl = nullptr, *dpl2 = nullptr, *adapt = nullptr, *dchi = nullptr, *stage = nullptr;
     int *counters = nullptr;
+    stz::HostRing ring;         // copies of whole fields to and from the caller's memory
     // direct (explicit dynamics) step: reference map and its double buffer,
     // second velocity buffer; allocated by the first direct-step call
     double *xi = nullptr, *xi2 = nullptr, *vel2 = nullptr;

@@ -156,9 +156,8 @@ int cube_size(const stz_t s, int mode, long *n) {
             return stz_detail::fail((s), STZMG_ERR_HIP, "%s: %s", #call, hipGetErrorString(e_)); \
     } while (0)
 
-int cube_host(stz_t s, int mode, std::vector<float> &h) {
-    long n = 0;
-    if (int rc = cube_size(s, mode, &n)) return rc;
+// The cube's n values (cube_size) into host memory.
+int cube_host(stz_t s, int mode, long n, float *h) {
     const Grid &g = s->g;
     const int nzo = (int)(n / ((long)g.Nx * g.Ny));
     float *d = reinterpret_cast<float *>(s->stage);  // 6 max(Nc, Nv) doubles: room for any cube
@@ -166,9 +165,7 @@ int cube_host(stz_t s, int mode, std::vector<float> &h) {
                        s->stream, g, mode, nzo, (const double *)s->vel, (const double *)s->sig,
                        (const double *)s->chi, (const double *)s->xi, s->p.bz - s->p.az, d);
     OHIP(s, hipGetLastError());
-    h.resize(n);
-    OHIP(s, hipMemcpyAsync(h.data(), d, sizeof(float) * n, hipMemcpyDeviceToHost, s->stream));
-    OHIP(s, hipStreamSynchronize(s->stream));
+    OHIP(s, s->ring.download(h, d, sizeof(float) * n, s->stream));
     return 0;
 }
 
@@ -230,8 +227,10 @@ int write_traction(stz_t s, const char *dir) {
 
 int write_cube(stz_t s, const char *dir, const char *name, int mode, int frame) {
     if (int rc = ensure_dir(s, dir)) return rc;
-    std::vector<float> h;
-    if (int rc = cube_host(s, mode, h)) return rc;
+    long n = 0;
+    if (int rc = cube_size(s, mode, &n)) return rc;
+    std::vector<float> h(n);
+    if (int rc = cube_host(s, mode, n, h.data())) return rc;
     char path[4096];
     snprintf(path, sizeof(path), "%s/%s_grid.%d", dir, name, frame);
     return append(s, path, h.data(), sizeof(float) * h.size());
@@ -267,10 +266,7 @@ int stz_output_cube(stz_t s, int mode, float *out, long long n) {
     if (int rc = cube_size(s, mode, &need)) return rc;
     if (!out) return (int)STZMG_ERR_ARG;
     if (n < need) return stz_detail::fail(s, STZMG_ERR_ARG, "cube needs %ld values, buffer holds %lld", need, n);
-    std::vector<float> h;
-    if (int rc = cube_host(s, mode, h)) return rc;
-    memcpy(out, h.data(), sizeof(float) * h.size());
-    return 0;
+    return cube_host(s, mode, need, out);
 }
 
 long long stz_cube_size(stz_t s, int mode) {
