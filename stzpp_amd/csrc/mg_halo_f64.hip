@@ -1,4 +1,4 @@
-// Instances of the one-launch sweep (mg_instances.hpp).
+// Instances of the small levels' one-launch kernels (mg_instances.hpp).
 #include "mg_instances.hpp"
 
 namespace stzmg {

@@ -8,6 +8,7 @@
 #include "mg_halo.hpp"
 #include "mg_march.hpp"
 #include "mg_resid.hpp"
+#include "mg_restrict.hpp"
 
 namespace stzmg {
 
@@ -82,9 +83,13 @@ constexpr int kHaloTile = 8;
     STZ_SWEEP_INST(PRE, T, 4) STZ_SWEEP_INST(PRE, T, 5) STZ_SWEEP_INST(PRE, T, 6) STZ_SWEEP_INST(PRE, T, 7)
 
 #define STZ_HALO_SIG(T) \
-    (Dims, const T *__restrict__, T *__restrict__, const T *__restrict__, const T *__restrict__, int)
-#define STZ_HALO_INST(PRE, T, KEY) \
-    PRE template __global__ void k_gs_halo<T, KEY, kHaloTile, kHaloTile> STZ_HALO_SIG(T);
+    (Dims, const T *__restrict__, T *__restrict__, const T *__restrict__, const T *__restrict__, int, Dims, \
+     const T *__restrict__)
+#define STZ_RR_SIG(T) \
+    (Dims, Dims, const T *__restrict__, const T *__restrict__, const T *__restrict__, T *__restrict__, T *__restrict__)
+#define STZ_HALO_INST(PRE, T, KEY)                                                        \
+    PRE template __global__ void k_gs_halo<T, KEY, kHaloTile, kHaloTile> STZ_HALO_SIG(T); \
+    PRE template __global__ void k_resid_restrict<T, KEY> STZ_RR_SIG(T);
 #define STZ_HALO_PLAIN(PRE, T) \
     STZ_HALO_INST(PRE, T, 0) STZ_HALO_INST(PRE, T, 1) STZ_HALO_INST(PRE, T, 2) STZ_HALO_INST(PRE, T, 3)
 #define STZ_HALO_SYM(PRE, T) \
@@ -100,7 +105,8 @@ constexpr int kHaloTile = 8;
     STZ_RESID_ONE(PRE, T, KEY, false, false, ResidTile<T>::TX, ResidTile<T>::TY)     \
     STZ_RESID_ONE(PRE, T, KEY, false, true, ResidTile<T>::TX, ResidTile<T>::TY)      \
     STZ_RESID_ONE(PRE, T, KEY, false, false, kResidSmall, kResidSmall)               \
-    STZ_RESID_ONE(PRE, T, KEY, false, true, kResidSmall, kResidSmall)
+    STZ_RESID_ONE(PRE, T, KEY, false, true, kResidSmall, kResidSmall)                \
+    STZ_RESID_ONE(PRE, T, KEY, true, false, kResidSmall, kResidSmall)
 #define STZ_RESID_ALL(PRE, T)                                                                                \
     STZ_RESID_INST(PRE, T, 0) STZ_RESID_INST(PRE, T, 1) STZ_RESID_INST(PRE, T, 2) STZ_RESID_INST(PRE, T, 3)  \
     STZ_RESID_INST(PRE, T, 4) STZ_RESID_INST(PRE, T, 5) STZ_RESID_INST(PRE, T, 6) STZ_RESID_INST(PRE, T, 7)

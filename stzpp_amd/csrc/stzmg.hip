@@ -46,7 +46,8 @@ struct Level {
     float *x32b = nullptr;
     bool fused = false;   // fused two-launch sweeps on this level
     bool tiled = false;   // LDS plane-marching residual on this level
-    bool tiled_small = false;  // the same with the small tiles (no norm partials)
+    bool tiled_small = false;  // the same with the small tiles
+    bool rr = false;      // residual and restriction in one launch (mg_restrict.hpp)
     int ftile = 0;        // fused-smoother tile class of FP32 sweeps (fused_tile)
     int ftile64 = 0;      // and of FP64 sweeps
     int pat = 0;          // operator zero pattern (PAT_*)
@@ -231,11 +232,24 @@ bool tiled_ok(const Level &L) {
 
 // Smaller tiles of the marching residual (16 x 16, one point per thread) for
 // plane levels periodic in x and y that the tiles above do not divide (the
-// 96^2 and 48^2 levels of a 192^2 grid, 32^3 and 16^3 below 256^3); used for
-// the V-cycle's residuals, which take no norm partials.
+// 96^2 and 48^2 levels of a 192^2 grid, 32^3 and 16^3 below 256^3).  With
+// norm partials 32 x 32 x 33 takes 5 us (13.8 with one thread per point).
 bool tiled_small_ok(const Level &L) {
     return L.mode == STZMG_OP_PLANE && L.d.px && L.d.py && !tiled_ok(L) && L.d.m % kResidSmall == 0 &&
            L.d.n % kResidSmall == 0;
+}
+
+// Residual and restriction in one launch (k_resid_restrict): plane levels up
+// to kRRMaxPoints.  Below, the two launches are latency and one saves about
+// 6 us a V-cycle and level (one V-cycle FP64 / FP32, two launches against
+// one: 32 x 32 x 33 150 / 133 -> 137 / 121 us; 64 x 64 x 65 with its 266,240
+// points 292 / 251 -> 280 / 240; 96 x 80 x 49, 376,320, 360 / 308 -> 334 /
+// 284); at 128 x 128 x 65 (1,064,960) the residuals computed twice cost more
+// than the launch (558 / 445 -> 571 / 457).
+constexpr long kRRMaxPoints = 400000;
+bool rr_ok(const Level &L) {
+    return L.mode == STZMG_OP_PLANE && L.d.px && L.d.py && L.d.m % 2 == 0 && L.d.n % 2 == 0 && L.d.m >= 8 &&
+           L.d.n >= 8 && L.d.N <= kRRMaxPoints;
 }
 
 // Workgroups of the plane-marching residual in type T resident on the
@@ -284,6 +298,29 @@ dim3 tiled_grid(const Level &L, long cap, int *kchunk, bool norm) {
     return dim3(L.d.m / ResidTile<T>::TX, L.d.n / ResidTile<T>::TY, (L.d.o + kc - 1) / kc);
 }
 
+// Grid of the small-tile residual: z chunks for about 1024 workgroups (a
+// fixed number: the norm partials do not depend on the device).
+dim3 resid_small_grid(const Level &L, int *kchunk) {
+    const long tiles = (long)(L.d.m / kResidSmall) * (L.d.n / kResidSmall);
+    const long nz = std::min<long>(L.d.o, std::max<long>(1, 1024 / tiles));
+    const int kc = (int)((L.d.o + nz - 1) / nz);
+    *kchunk = kc;
+    return dim3(L.d.m / kResidSmall, L.d.n / kResidSmall, (L.d.o + kc - 1) / kc);
+}
+
+template <typename T, bool NORM, bool APPLY, int PAT>
+void launch_resid_small(stzmg_t h, Level &L, const T *x, const T *r, T *out, T *xcopy, double *part) {
+    int kc;
+    const dim3 g = resid_small_grid(L, &kc);
+    constexpr int S = kResidSmall;
+    if (L.sym)
+        hipLaunchKernelGGL((k_resid_march<T, PAT + kMarchSym, NORM, APPLY, S, S, kThreads>), g, dim3(kThreads), 0,
+                           h->stream, L.d, x, r, (const T *)pkr_of<T>(L), out, part, kc, xcopy);
+    else
+        hipLaunchKernelGGL((k_resid_march<T, PAT, NORM, APPLY, S, S, kThreads>), g, dim3(kThreads), 0, h->stream,
+                           L.d, x, r, (const T *)pkr_of<T>(L), out, part, kc, xcopy);
+}
+
 // Number of norm partials the residual of level L writes.
 template <typename T>
 long resid_parts(stzmg_t h, const Level &L) {
@@ -292,23 +329,12 @@ long resid_parts(stzmg_t h, const Level &L) {
         const dim3 g = tiled_grid<T>(L, h->chunk_cap, &kc, true);
         return (long)g.x * g.y * g.z;
     }
+    if (L.tiled_small) {
+        int kc;
+        const dim3 g = resid_small_grid(L, &kc);
+        return (long)g.x * g.y * g.z;
+    }
     return (long)nblk((long)L.d.m * L.d.n) * L.d.o;
-}
-
-template <typename T, bool APPLY, int PAT>
-void launch_resid_small(stzmg_t h, Level &L, const T *x, const T *r, T *out, T *xcopy) {
-    // z chunks: about 1024 workgroups
-    const long tiles = (long)(L.d.m / kResidSmall) * (L.d.n / kResidSmall);
-    const long nz = std::min<long>(L.d.o, std::max<long>(1, 1024 / tiles));
-    const int kc = (int)((L.d.o + nz - 1) / nz);
-    dim3 g(L.d.m / kResidSmall, L.d.n / kResidSmall, (L.d.o + kc - 1) / kc);
-    constexpr int S = kResidSmall;
-    if (L.sym)
-        hipLaunchKernelGGL((k_resid_march<T, PAT + kMarchSym, false, APPLY, S, S, kThreads>), g, dim3(kThreads), 0,
-                           h->stream, L.d, x, r, (const T *)pkr_of<T>(L), out, (double *)nullptr, kc, xcopy);
-    else
-        hipLaunchKernelGGL((k_resid_march<T, PAT, false, APPLY, S, S, kThreads>), g, dim3(kThreads), 0, h->stream,
-                           L.d, x, r, (const T *)pkr_of<T>(L), out, (double *)nullptr, kc, xcopy);
 }
 
 template <typename T, bool NORM, bool APPLY, int PAT>
@@ -340,12 +366,12 @@ void launch_resid_any(stzmg_t h, Level &L, const T *x, const T *r, T *out, T *xc
         }
         return;
     }
-    if (!NORM && L.tiled_small) {
+    if (L.tiled_small) {
         switch (L.pat) {
-            case PAT_SHEAR: launch_resid_small<T, APPLY, PAT_SHEAR>(h, L, x, r, out, xcopy); break;
-            case PAT_TRANS_XZ: launch_resid_small<T, APPLY, PAT_TRANS_XZ>(h, L, x, r, out, xcopy); break;
-            case PAT_NOCORNER: launch_resid_small<T, APPLY, PAT_NOCORNER>(h, L, x, r, out, xcopy); break;
-            default: launch_resid_small<T, APPLY, PAT_DENSE>(h, L, x, r, out, xcopy); break;
+            case PAT_SHEAR: launch_resid_small<T, NORM, APPLY, PAT_SHEAR>(h, L, x, r, out, xcopy, part); break;
+            case PAT_TRANS_XZ: launch_resid_small<T, NORM, APPLY, PAT_TRANS_XZ>(h, L, x, r, out, xcopy, part); break;
+            case PAT_NOCORNER: launch_resid_small<T, NORM, APPLY, PAT_NOCORNER>(h, L, x, r, out, xcopy, part); break;
+            default: launch_resid_small<T, NORM, APPLY, PAT_DENSE>(h, L, x, r, out, xcopy, part); break;
         }
         return;
     }
@@ -499,7 +525,7 @@ void launch_fused_tile(stzmg_t h, Level &L, bool zero_start = false) {
 
 // One sweep in one launch (mg_halo.hpp).
 template <typename T, int KEY>
-void launch_halo(stzmg_t h, Level &L, bool zero_start) {
+void launch_halo(stzmg_t h, Level &L, bool zero_start, const Level *corr) {
     const Dims &d = L.d;
     constexpr int TX = kHaloTile;
     T *x = xref_of<T>(L), *xb = xb_of<T>(L);
@@ -507,7 +533,8 @@ void launch_halo(stzmg_t h, Level &L, bool zero_start) {
     const bool rec = h->launch_ev && h->launch_ev_next + 2 <= h->launch_ev->size();
     if (rec) (void)hipEventRecord((*h->launch_ev)[h->launch_ev_next], h->stream);
     hipLaunchKernelGGL((k_gs_halo<T, KEY, TX, TX>), g, dim3(halo_threads<TX, TX>()), 0, h->stream, d, (const T *)x, xb,
-                       (const T *)r_of<T>(L), (const T *)pk_of<T>(L), zero_start ? 1 : 0);
+                       (const T *)r_of<T>(L), (const T *)pk_of<T>(L), zero_start ? 1 : 0, corr ? corr->d : d,
+                       corr ? (const T *)x_of<T>(const_cast<Level &>(*corr)) : (const T *)nullptr);
     if (rec) {
         (void)hipEventRecord((*h->launch_ev)[h->launch_ev_next + 1], h->stream);
         h->launch_ev_next += 2;
@@ -516,11 +543,11 @@ void launch_halo(stzmg_t h, Level &L, bool zero_start) {
 }
 
 template <typename T, int PAT>
-void launch_fused_pat(stzmg_t h, Level &L, bool zero_start) {
+void launch_fused_pat(stzmg_t h, Level &L, bool zero_start, const Level *corr) {
     const int ft = sizeof(T) == 4 ? L.ftile : L.ftile64;
     if (ft == 4) {
-        if (L.sym) launch_halo<T, PAT + kMarchSym>(h, L, zero_start);
-        else launch_halo<T, PAT>(h, L, zero_start);
+        if (L.sym) launch_halo<T, PAT + kMarchSym>(h, L, zero_start, corr);
+        else launch_halo<T, PAT>(h, L, zero_start, corr);
         return;
     }
     if (ft == 1) {
@@ -561,22 +588,25 @@ void launch_gs_sweep_colours(stzmg_t h, Level &L);
 
 // Whether a sweep of level L can start from x = 0 without the zeros in
 // memory (the fused sweep k_gs_march skips the planes it knows are zero).
+template <typename T>
+bool correction_ok(const Level &L) { return L.fused && (sizeof(T) == 4 ? L.ftile : L.ftile64) == 4; }
 bool zero_start_ok(const Level &L) { return STZ_MARCH != 0 && L.fused; }
 
 // One Gauss-Seidel sweep of a level: one or two fused launches where the
 // level allows, eight colour launches otherwise.  zero_start (only where
-// zero_start_ok): the sweep starts from x = 0 whatever x holds.
+// zero_start_ok): the sweep starts from x = 0 whatever x holds.  corr (only
+// where correction_ok): it starts from x + P x of that coarse level.
 template <typename T>
-void launch_gs_sweep(stzmg_t h, Level &L, bool zero_start = false) {
+void launch_gs_sweep(stzmg_t h, Level &L, bool zero_start = false, const Level *corr = nullptr) {
     if (!L.fused) {
         launch_gs_sweep_colours<T>(h, L);
         return;
     }
     switch (L.pat) {
-        case PAT_SHEAR: launch_fused_pat<T, PAT_SHEAR>(h, L, zero_start); break;
-        case PAT_TRANS_XZ: launch_fused_pat<T, PAT_TRANS_XZ>(h, L, zero_start); break;
-        case PAT_NOCORNER: launch_fused_pat<T, PAT_NOCORNER>(h, L, zero_start); break;
-        default: launch_fused_pat<T, PAT_DENSE>(h, L, zero_start); break;
+        case PAT_SHEAR: launch_fused_pat<T, PAT_SHEAR>(h, L, zero_start, corr); break;
+        case PAT_TRANS_XZ: launch_fused_pat<T, PAT_TRANS_XZ>(h, L, zero_start, corr); break;
+        case PAT_NOCORNER: launch_fused_pat<T, PAT_NOCORNER>(h, L, zero_start, corr); break;
+        default: launch_fused_pat<T, PAT_DENSE>(h, L, zero_start, corr); break;
     }
 }
 
@@ -615,10 +645,32 @@ void launch_gs_sweep_colours(stzmg_t h, Level &L) {
             }
 }
 
+template <typename T, int PAT>
+void launch_resid_restrict(stzmg_t h, Level &F, Level &C) {
+    const dim3 g((C.d.m + kRR - 1) / kRR, (C.d.n + kRR - 1) / kRR, C.d.o);
+    if (F.sym)
+        hipLaunchKernelGGL((k_resid_restrict<T, PAT + kMarchSym>), g, dim3(kRRThreads), 0, h->stream, F.d, C.d,
+                           (const T *)x_of<T>(F), (const T *)r_of<T>(F), (const T *)pkr_of<T>(F), r_of<T>(C),
+                           x_of<T>(C));
+    else
+        hipLaunchKernelGGL((k_resid_restrict<T, PAT>), g, dim3(kRRThreads), 0, h->stream, F.d, C.d,
+                           (const T *)x_of<T>(F), (const T *)r_of<T>(F), (const T *)pkr_of<T>(F), r_of<T>(C),
+                           x_of<T>(C));
+}
+
 // Level l (coarse) receives the restricted residual of level l-1.
 template <typename T>
 void launch_restrict(stzmg_t h, int l) {
     Level &F = h->lv[l - 1], &C = h->lv[l];
+    if (F.rr) {
+        switch (F.pat) {
+            case PAT_SHEAR: launch_resid_restrict<T, PAT_SHEAR>(h, F, C); break;
+            case PAT_TRANS_XZ: launch_resid_restrict<T, PAT_TRANS_XZ>(h, F, C); break;
+            case PAT_NOCORNER: launch_resid_restrict<T, PAT_NOCORNER>(h, F, C); break;
+            default: launch_resid_restrict<T, PAT_DENSE>(h, F, C); break;
+        }
+        return;
+    }
     launch_resid<T, false>(h, F, x_of<T>(F), r_of<T>(F), t_of<T>(F));
     if (F.d.px && F.d.py && C.d.m % kRestrictTX == 0 && C.d.n % kRestrictTY == 0) {
         // LDS-staged tiles; coarse planes per workgroup: as many as keep
@@ -781,8 +833,11 @@ void enqueue_vcycle(stzmg_t h, bool zero_top = false) {
         }
     }
     for (int i = top; i > 0; i--) {
-        launch_interp<T>(h, i);
-        for (int q = 0; q < sweeps_up(h, i - 1); q++) launch_gs_sweep<T>(h, h->lv[i - 1]);
+        // a one-launch sweep adds the correction itself
+        const bool own = sweeps_up(h, i - 1) > 0 && correction_ok<T>(h->lv[i - 1]);
+        if (!own) launch_interp<T>(h, i);
+        for (int q = 0; q < sweeps_up(h, i - 1); q++)
+            launch_gs_sweep<T>(h, h->lv[i - 1], false, own && q == 0 ? &h->lv[i] : nullptr);
     }
     for (int i = 0; i < L; i++) restore_level<T>(h, h->lv[i], home[i]);
     if (sizeof(T) == 4) restore_level<double>(h, h->lv[L - 1], home_b64);
@@ -968,7 +1023,7 @@ int pack_march(stzmg_t h) {
         const long n = L.ncls * stride;
         // the marching residual's tables, wherever it may run (the tiled
         // residual can be switched on after the operator is set)
-        if (tiled_ok(L) || tiled_small_ok(L)) {
+        if (tiled_ok(L) || tiled_small_ok(L) || rr_ok(L)) {
             const int *mapr = h->pkrmap + (long)key * kPackMax;
             if (!L.pkr32) HIPCHK(h, alloc(&L.pkr32, L.ncls * kPackMax));
             if (!L.pkr64) HIPCHK(h, alloc(&L.pkr64, L.ncls * kPackMax));
@@ -1057,7 +1112,7 @@ int build_hierarchy_ops(stzmg_t h) {
     // kernel configuration (an operator that changes every step, as in the
     // transformed step, then keeps its graphs).
     auto config = [](const Level &L) {
-        return std::make_tuple(L.fused, L.tiled, L.tiled_small, L.ftile, L.ftile64, L.pat, L.sym);
+        return std::make_tuple(L.fused, L.tiled, L.tiled_small, L.rr, L.ftile, L.ftile64, L.pat, L.sym);
     };
     std::vector<decltype(config(h->lv[0]))> before;
     for (auto &L : h->lv) before.push_back(config(L));
@@ -1069,6 +1124,7 @@ int build_hierarchy_ops(stzmg_t h) {
         L.fused = false;
         L.tiled = false;
         L.tiled_small = false;
+        L.rr = false;
         if (L.mode != STZMG_OP_PLANE) continue;
         const unsigned *used = cfg.data() + l * kCfgWords;  // per block: entries nonzero on some plane
         int pat = PAT_DENSE;
@@ -1089,6 +1145,7 @@ int build_hierarchy_ops(stzmg_t h) {
         L.fused = h->fused_smoother && L.ftile && L.ftile64 && L.x64b;
         L.tiled = h->tiled_resid && tiled_ok(L);
         L.tiled_small = h->tiled_resid && tiled_small_ok(L);
+        L.rr = h->tiled_resid && l + 1 < h->lv.size() && rr_ok(L);
     }
     if (int rc = pack_march(h)) return rc;
     bool same = h->ops_set;
@@ -1304,6 +1361,7 @@ int stzmg_set_option(stzmg_t h, int option, int value) {
         for (auto &L : h->lv) {
             L.tiled = h->ops_set && h->tiled_resid && tiled_ok(L);
             L.tiled_small = h->ops_set && h->tiled_resid && tiled_small_ok(L);
+            L.rr = h->ops_set && h->tiled_resid && &L != &h->lv.back() && rr_ok(L);
         }
     } else if (option == STZMG_OPT_BOTTOM_MAP) {
         h->bottom_map = value != 0;

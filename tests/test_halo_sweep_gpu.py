@@ -101,3 +101,29 @@ def test_vcycle_from_zero(m, n, o, pz):
     mg.v_cycle(2)
     orc.vcycle(2)
     assert relerr(mg.x(0), orc.fields(0)[0]) < 1e-11
+
+
+@pytest.mark.parametrize("m,n,o,pz", [(8, 16, 16, 1), (12, 20, 9, 0), (16, 16, 17, 0), (18, 22, 13, 0), (32, 24, 16, 1),
+                                      (36, 44, 25, 0), (64, 64, 33, 0)])
+@pytest.mark.parametrize("kind", ["shear", "trans", "full", "dense", "plain"])
+def test_residual_and_restriction_in_one_launch(kind, m, n, o, pz):
+    """Tiles that stick out of the coarse plane, one and several tiles, walls
+    and periodic z; the residual is a 27-block sum and the restriction 27
+    weights, so FP64 rounding stays below 1e-12 of the largest value."""
+    prd = (1, 1, pz)
+    planes = planes_of(kind, m, n, o, pz)
+    N = m * n * o
+    x, r = O.det_field(N, 51), O.det_field(N, 52)
+    mg = MG.Multigrid(m, n, o, prd, coarsest_total=N - 1)
+    mg.setup_matrices_planes(planes)
+    orc = O.OracleMG(m, n, o, prd, mode=O.PLANE, coarsest_total=N - 1)
+    orc.set_ops(0, planes)
+    assert mg.nlevels == 2
+    mg.setup_fields(x, r)
+    mg.setup_fields(O.det_field(mg.npts(1), 53), None, 1)
+    orc.set_fields(0, x, r)
+    mg.restriction(1)
+    orc.restrict(1)
+    xc, rc = mg.fields(1)
+    assert not xc.any()
+    assert relerr(rc, orc.fields(1)[1]) < 1e-12
