@@ -70,12 +70,12 @@ __global__ __launch_bounds__(kThreads) void k_mdot(const TV *__restrict__ w, con
     }
 }
 
-// w -= sum_j coef[j] V_j (j < NV) in FP64, stored as TV, then part[b] =
-// block share of |w|^2 (of the stored values).
+// w -= sum_j coef[j] V_j (j < NV) in FP64, stored as TV (also to copy unless
+// null), then part[b] = block share of |w|^2 (of the stored values).
 template <int NV, typename TV = double>
 __global__ __launch_bounds__(kThreads) void k_maxpy_norm(TV *__restrict__ w, const TV *__restrict__ V,
                                                          const double *__restrict__ coef, long n3,
-                                                         double *__restrict__ part) {
+                                                         double *__restrict__ part, TV *__restrict__ copy) {
     double c[NV];
 #pragma unroll
     for (int j = 0; j < NV; j++) c[j] = coef[j];
@@ -99,6 +99,7 @@ __global__ __launch_bounds__(kThreads) void k_maxpy_norm(TV *__restrict__ w, con
             for (int j = 0; j < NV; j++) wi -= c[j] * (double)vv[u][j];
             const TV ws = (TV)wi;
             w[i + u * S] = ws;
+            if (copy) copy[i + u * S] = ws;
             acc += (double)ws * (double)ws;
         }
     }
@@ -108,6 +109,7 @@ __global__ __launch_bounds__(kThreads) void k_maxpy_norm(TV *__restrict__ w, con
         for (int j = 0; j < NV; j++) wi -= c[j] * (double)V[(long)j * n3 + i];
         const TV ws = (TV)wi;
         w[i] = ws;
+        if (copy) copy[i] = ws;
         acc += (double)ws * (double)ws;
     }
     __shared__ double red[kThreads / 64];
@@ -134,22 +136,31 @@ void launch_mdot_n(hipStream_t st, const TV *w, const TV *V, int nv, long n3, do
     }
 }
 template <int NV, typename TV = double>
-void launch_maxpy_n(hipStream_t st, TV *w, const TV *V, const double *coef, int nv, long n3, double *part) {
+void launch_maxpy_n(hipStream_t st, TV *w, const TV *V, const double *coef, int nv, long n3, double *part,
+                    TV *copy = nullptr) {
     if constexpr (NV <= kKrylovMax + 1) {
         if (nv == NV) {
             hipLaunchKernelGGL((k_maxpy_norm<NV, TV>), dim3(kDotBlocks), dim3(kThreads), 0, st, w, V, coef, n3,
-                               part);
+                               part, copy);
             return;
         }
-        launch_maxpy_n<NV + 1, TV>(st, w, V, coef, nv, n3, part);
+        launch_maxpy_n<NV + 1, TV>(st, w, V, coef, nv, n3, part, copy);
     }
 }
 
-// out[j] = sum_b part[b * nv + j] (one block per column, fixed order),
-// times scale[j] when scale is given.
-__global__ __launch_bounds__(kThreads) void k_reduce_cols(const double *__restrict__ part, int nblocks, int nv,
-                                                          double *__restrict__ out,
-                                                          const double *__restrict__ scale) {
+// One value per Krylov vector, passed to a kernel by value (no copy of its
+// own in the stream).
+struct KrylovVals {
+    double v[kKrylovMax + 1];
+};
+
+// sum_b part[b * nv + j] (one block per column j, fixed order), times
+// scale.v[j] when scaled, to out[j] (device, unless null) and host[j]: pinned
+// host memory, written by the kernel itself, so that the host reads it after
+// its synchronization without a copy in between.
+static __global__ __launch_bounds__(kThreads) void k_reduce_cols(const double *__restrict__ part, int nblocks, int nv,
+                                                          double *__restrict__ out, double *__restrict__ host,
+                                                          int scaled, KrylovVals scale) {
     const int j = blockIdx.x;
     double t = 0;
     for (int b = threadIdx.x; b < nblocks; b += kThreads) t += part[(long)b * nv + j];
@@ -160,14 +171,18 @@ __global__ __launch_bounds__(kThreads) void k_reduce_cols(const double *__restri
         if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[j] = scale ? red[0] * scale[j] : red[0];
+    if (threadIdx.x == 0) {
+        const double v = scaled ? red[0] * scale.v[j] : red[0];
+        if (out) out[j] = v;
+        host[j] = v;
+    }
 }
 
-// dst = a src (in FP64, stored as TD; kEW elements per thread, grid
-// nblk_ew(n3)).
+// dst = a src (in FP64, stored as TD, also to copy unless null; kEW elements
+// per thread, grid nblk_ew(n3)).
 template <typename TD = double, typename TS = double>
 __global__ __launch_bounds__(kThreads) void k_scale(TD *__restrict__ dst, const TS *__restrict__ src, double a,
-                                                    long n3) {
+                                                    long n3, TD *__restrict__ copy = nullptr) {
     const long b0 = (long)blockIdx.x * (kThreads * kEW) + threadIdx.x;
     TS v[kEW];
 #pragma unroll
@@ -178,7 +193,10 @@ __global__ __launch_bounds__(kThreads) void k_scale(TD *__restrict__ dst, const 
 #pragma unroll
     for (int u = 0; u < kEW; u++) {
         const long i = b0 + (long)u * kThreads;
-        if (i < n3) dst[i] = (TD)(a * (double)v[u]);
+        if (i < n3) {
+            dst[i] = (TD)(a * (double)v[u]);
+            if (copy) copy[i] = (TD)(a * (double)v[u]);
+        }
     }
 }
 
@@ -186,8 +204,8 @@ __global__ __launch_bounds__(kThreads) void k_scale(TD *__restrict__ dst, const 
 // The loads of one basis vector for all kEW elements are issued together;
 // each element's terms are added in the order j = 0, 1, ...
 template <typename TZ = float>
-__global__ __launch_bounds__(kThreads) void k_xupdate(double *__restrict__ x, const TZ *__restrict__ Z,
-                                                      const double *__restrict__ y, int nv, long n3) {
+__global__ __launch_bounds__(kThreads) void k_xupdate(double *__restrict__ x, const TZ *__restrict__ Z, KrylovVals y,
+                                                      int nv, long n3) {
     const long b0 = (long)blockIdx.x * (kThreads * kEW) + threadIdx.x;
     double s[kEW];
 #pragma unroll
@@ -196,7 +214,7 @@ __global__ __launch_bounds__(kThreads) void k_xupdate(double *__restrict__ x, co
         s[u] = i < n3 ? x[i] : 0.0;
     }
     for (int j = 0; j < nv; j++) {
-        const double yj = y[j];
+        const double yj = y.v[j];
         const TZ *Zj = Z + (long)j * n3;
         TZ z[kEW];
 #pragma unroll

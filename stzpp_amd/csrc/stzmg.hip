@@ -101,11 +101,10 @@ struct stzmg_s {
     std::string err;
     double *part = nullptr;   // per-block norm partials
     long part_cap = 0;
-    double *dres = nullptr;   // reduced norms (2 doubles)
     int *dflag = nullptr;     // singular-block flag
     unsigned *dcfg = nullptr; // k_level_config words of every level
-    double *hres = nullptr;   // pinned host copy of dres (reference loop)
-    hipEvent_t evres = nullptr;  // recorded after that copy
+    double *hres = nullptr;   // pinned host memory the reductions write: a norm pair, then a Krylov column
+    hipEvent_t evres = nullptr;  // recorded after that norm (reference loop)
     bool ops_set = false;
     int std_iters = 16;       // per-handle copy of the reference's static heuristic
     long coarse_max = kCoarseMaxPoints;  // levels this small run in one workgroup (0: off)
@@ -860,27 +859,26 @@ int norms64(stzmg_t h, int l, double out[2]) {
     if (ensure_part(h, nb)) return STZMG_ERR_NOMEM;
     launch_resid<double, true>(h, L, L.x64, L.r64, L.t64);
     hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, h->stream, (const double *)h->part, nb,
-                       h->dres);
+                       h->hres);
     LAUNCHCHK(h);
-    HIPCHK(h, hipMemcpyAsync(out, h->dres, 2 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    out[0] = h->hres[0];
+    out[1] = h->hres[1];
     return 0;
 }
 
-// The same norms, enqueued: the reduced pair is copied to the pinned h->hres
-// and h->evres recorded after the copy; the caller may enqueue more work
-// and then wait on the event.
+// The same norms, enqueued: the reduced pair goes to the pinned h->hres and
+// h->evres is recorded after it; the caller may enqueue more work and then
+// wait on the event.
 int norms64_enqueue(stzmg_t h, int l) {
     Level &L = h->lv[l];
     const long nb = resid_parts<double>(h, L);
     if (ensure_part(h, nb)) return STZMG_ERR_NOMEM;
-    if (!h->hres) HIPCHK(h, hipHostMalloc((void **)&h->hres, 2 * sizeof(double), hipHostMallocDefault));
     if (!h->evres) HIPCHK(h, hipEventCreateWithFlags(&h->evres, hipEventDisableTiming));
     launch_resid<double, true>(h, L, L.x64, L.r64, L.t64);
     hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, h->stream, (const double *)h->part, nb,
-                       h->dres);
+                       h->hres);
     LAUNCHCHK(h);
-    HIPCHK(h, hipMemcpyAsync(h->hres, h->dres, 2 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipEventRecord(h->evres, h->stream));
     return 0;
 }
@@ -893,10 +891,11 @@ int norms64_of(stzmg_t h, int l, const double *x, const double *r, double out[2]
     if (ensure_part(h, nb)) return STZMG_ERR_NOMEM;
     launch_resid<double, true>(h, L, x, r, L.t64);
     hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, h->stream, (const double *)h->part, nb,
-                       h->dres);
+                       h->hres);
     LAUNCHCHK(h);
-    HIPCHK(h, hipMemcpyAsync(out, h->dres, 2 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    out[0] = h->hres[0];
+    out[1] = h->hres[1];
     return 0;
 }
 
@@ -926,7 +925,7 @@ int ensure_krylov(stzmg_t h, int m, long n3, bool basis64) {
         h->kcap = 0;
         HIPCHK(h, alloc(&h->kZ, (long)m * n3));
         HIPCHK(h, alloc(&h->kpart, (long)kDotBlocks * (kKrylovMax + 1)));
-        HIPCHK(h, alloc(&h->kdev, 2L * (kKrylovMax + 1)));
+        HIPCHK(h, alloc(&h->kdev, kKrylovMax + 1));
         h->kcap = m;
     }
     if (basis64 && h->kcap64 < m) {
@@ -1227,6 +1226,8 @@ int stzmg_create(const stzmg_desc *d, stzmg_t *out) {
     auto bail = [&](int code) {
         g_create_err = h->err;
         for (auto &L : h->lv) free_level(L);
+        hipFree(h->dflag);
+        if (h->hres) hipHostFree(h->hres);
         if (h->stream) hipStreamDestroy(h->stream);
         delete h;
         return code;
@@ -1292,7 +1293,9 @@ int stzmg_create(const stzmg_desc *d, stzmg_t *out) {
         hipMemsetAsync(L.x32, 0, sizeof(float) * n3, h->stream);
         hipMemsetAsync(L.r32, 0, sizeof(float) * n3, h->stream);
     }
-    if (alloc(&h->dres, 2) || alloc(&h->dflag, 1)) return bail(fail(h, STZMG_ERR_NOMEM, "allocation failed"));
+    if (alloc(&h->dflag, 1) || hipHostMalloc((void **)&h->hres, sizeof(double) * (2 + kKrylovMax + 2),
+                                             hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess)
+        return bail(fail(h, STZMG_ERR_NOMEM, "allocation failed"));
     if (hipStreamSynchronize(h->stream) != hipSuccess) return bail(fail(h, STZMG_ERR_HIP, "init sync failed"));
     *out = h;
     return 0;
@@ -1304,7 +1307,6 @@ int stzmg_destroy(stzmg_t h) {
     drop_graphs(h);
     for (auto &L : h->lv) free_level(L);
     hipFree(h->part);
-    hipFree(h->dres);
     hipFree(h->dflag);
     hipFree(h->dcfg);
     if (h->hres) hipHostFree(h->hres);
@@ -1661,6 +1663,7 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
     if (int rc = require_ops(h)) return rc;
     stzmg_solve_stats s{};
     const bool graph = opts->use_graph != 0;
+    double *hcol = h->hres + 2;  // Krylov column as the reductions leave it
     auto t0 = std::chrono::steady_clock::now();
     double v[2];
     int rc = 0;
@@ -1781,7 +1784,7 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
         const unsigned nb3 = nblk(n3);
         while (rc == 0 && s.res > target && beta > 0) {
             hipLaunchKernelGGL((k_scale<double, double>), dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, h->kV, (const double *)L.t64,
-                               1.0 / beta, n3);
+                               1.0 / beta, n3, (double *)nullptr);
             std::fill(g.begin(), g.end(), 0.0);
             g[0] = beta;
             int nj = 0;
@@ -1802,22 +1805,21 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
                 // d_i = (w', v_i); w' -= sum d_i v_i; |w'|^2
                 launch_mdot_n<1>(h->stream, (const double *)w, (const double *)h->kV, j + 1, n3, h->kpart);
                 hipLaunchKernelGGL(k_reduce_cols, dim3(j + 1), dim3(kThreads), 0, h->stream,
-                                   (const double *)h->kpart, kDotBlocks, j + 1, h->kdev, (const double *)nullptr);
+                                   (const double *)h->kpart, kDotBlocks, j + 1, h->kdev, hcol, 0, KrylovVals{});
                 launch_maxpy_n<1>(h->stream, w, (const double *)h->kV, (const double *)h->kdev, j + 1, n3,
                                   h->kpart);
                 hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(kThreads), 0, h->stream, (const double *)h->kpart,
-                                   kDotBlocks, 1, h->kdev + (j + 1), (const double *)nullptr);
+                                   kDotBlocks, 1, (double *)nullptr, hcol + (j + 1), 0, KrylovVals{});
                 LAUNCHCHK(h);
-                HIPCHK(h, hipMemcpyAsync(hc.data(), h->kdev, sizeof(double) * (j + 2), hipMemcpyDeviceToHost,
-                                         h->stream));
                 HIPCHK(h, hipStreamSynchronize(h->stream));
+                std::copy(hcol, hcol + j + 2, hc.begin());
                 const double wn = std::sqrt(hc[j + 1]);
                 for (int i = 0; i <= j; i++) Hc(i, j) = hc[i] / sigma;
                 Hc(j + 1, j) = wn / sigma;
                 if (!std::isfinite(wn)) { rc = STZMG_ERR_NONFINITE; break; }
                 if (wn > 0)
                     hipLaunchKernelGGL((k_scale<double, double>), dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, w, (const double *)w,
-                                       1.0 / wn, n3);
+                                       1.0 / wn, n3, (double *)nullptr);
                 // Givens rotations
                 for (int i = 0; i < j; i++) {
                     const double a = Hc(i, j), b = Hc(i + 1, j);
@@ -1841,10 +1843,10 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
                 for (int k2 = i + 1; k2 < nj; k2++) t -= Hc(i, k2) * y[k2];
                 y[i] = t / Hc(i, i);
             }
-            for (int i = 0; i < nj; i++) hc[i] = y[i] / sigma;
-            HIPCHK(h, hipMemcpyAsync(h->kdev, hc.data(), sizeof(double) * nj, hipMemcpyHostToDevice, h->stream));
+            KrylovVals yv{};
+            for (int i = 0; i < nj; i++) yv.v[i] = y[i] / sigma;
             hipLaunchKernelGGL(k_xupdate<float>, dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, L.x64, (const float *)h->kZ,
-                               (const double *)h->kdev, nj, n3);
+                               yv, nj, n3);
             LAUNCHCHK(h);
             s.outer++;
             if ((rc = norms64(h, 0, v))) return rc;
@@ -1866,9 +1868,13 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
         //
         // Basis vectors are kept unnormalised: u_j = nrm_j v_j.  The
         // reduction of the dot products scales (w, u_i) by 1/nrm_i^2, which
-        // gives the Gram-Schmidt coefficient of u_i directly, and the next
-        // defect scales u_j by sigma/nrm_j, so no separate normalisation pass
-        // runs.
+        // gives the Gram-Schmidt coefficient of u_i directly, and the
+        // preconditioner takes u_j as it is (z_j = M^-1 u_j; nrm_j enters the
+        // Hessenberg column and the update): the pass that forms u_j also
+        // writes it as the V-cycle's right-hand side, so neither a
+        // normalisation nor a defect pass runs (the defect pass took 91 us at
+        // 256^3).  u_j shrinks with the residual only, by at most the few
+        // orders a cycle gains, far from the limits of FP32.
         Level &L = h->lv[0];
         const long n3 = 3 * L.d.N;
         const int m = std::min(std::max(opts->restart, 1), kKrylovMax);
@@ -1880,54 +1886,49 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
         const double target = opts->rtol * beta;
         const double inner_rtol = opts->inner_rtol > 0 ? opts->inner_rtol : 1e-4;
         const int inner = opts->inner_cycles > 0 ? opts->inner_cycles : 1;
-        const double sigma = std::sqrt((double)n3);
         if (!std::isfinite(beta)) rc = STZMG_ERR_NONFINITE;
-        std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), g(m + 1), y(m), hc(m + 2), nrm(m + 1),
-            isq(kKrylovMax + 1);
+        std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), g(m + 1), y(m), hc(m + 2), nrm(m + 1);
         auto Hc = [&](int i, int j) -> double & { return H[(size_t)i * m + j]; };
         const unsigned nb3 = nblk(n3);
-        double *dscale = h->kdev + (kKrylovMax + 1);  // 1/nrm_i^2 on the device
+        KrylovVals isq{};  // 1/nrm_i^2
         while (rc == 0 && s.res > target && beta > 0) {
             hipLaunchKernelGGL((k_scale<float, double>), dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, h->kV32,
-                               (const double *)L.t64, 1.0 / beta, n3);
+                               (const double *)L.t64, 1.0 / beta, n3, L.r32);
             std::fill(g.begin(), g.end(), 0.0);
             g[0] = beta;
             nrm[0] = 1.0;
-            isq[0] = 1.0;
+            isq.v[0] = 1.0;
             const double stop = std::max(target, inner_rtol * beta);
             int nj = 0;
             for (int j = 0; j < m; j++) {
                 if (s.cycles >= opts->max_cycles) { rc = STZMG_ERR_NOT_CONVERGED; break; }
-                const float *uj = h->kV32 + (long)j * n3;
                 float *w = h->kV32 + (long)(j + 1) * n3;
                 float *zj = h->kZ + (long)j * n3;
-                // z_j = M^-1 (sigma v_j) = M^-1 (sigma / nrm_j u_j)
-                hipLaunchKernelGGL((k_defect_f32<float>), dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, uj,
-                                   sigma / nrm[j], L.r32, fine_zero_start(h) ? nullptr : L.x32, n3);
+                // z_j = M^-1 u_j, u_j in r32
+                if (!fine_zero_start(h))
+                    hipLaunchKernelGGL((k_fill<float>), dim3(nblk(n3)), dim3(kThreads), 0, h->stream, L.x32, 0.0f, n3);
                 if ((rc = run_vcycles<float>(h, inner, graph, true))) return rc;
                 s.cycles += inner;
-                // w' = A z_j in FP32 (the true w is w' / sigma); the same
+                // w' = A z_j in FP32 (A M^-1 v_j is w' / nrm_j); the same
                 // pass keeps z_j (x32 is overwritten by the next V-cycles)
                 launch_apply<float>(h, L, (const float *)L.x32, w, zj);
                 // c_i = (w', u_i) / nrm_i^2; w' -= sum c_i u_i; |w'|^2
-                HIPCHK(h, hipMemcpyAsync(dscale + j, &isq[j], sizeof(double), hipMemcpyHostToDevice, h->stream));
                 launch_mdot_n<1, float>(h->stream, (const float *)w, (const float *)h->kV32, j + 1, n3, h->kpart);
                 hipLaunchKernelGGL(k_reduce_cols, dim3(j + 1), dim3(kThreads), 0, h->stream,
-                                   (const double *)h->kpart, kDotBlocks, j + 1, h->kdev, (const double *)dscale);
+                                   (const double *)h->kpart, kDotBlocks, j + 1, h->kdev, hcol, 1, isq);
                 launch_maxpy_n<1, float>(h->stream, w, (const float *)h->kV32, (const double *)h->kdev, j + 1, n3,
-                                         h->kpart);
+                                         h->kpart, L.r32);
                 hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(kThreads), 0, h->stream, (const double *)h->kpart,
-                                   kDotBlocks, 1, h->kdev + (j + 1), (const double *)nullptr);
+                                   kDotBlocks, 1, (double *)nullptr, hcol + (j + 1), 0, KrylovVals{});
                 LAUNCHCHK(h);
-                HIPCHK(h, hipMemcpyAsync(hc.data(), h->kdev, sizeof(double) * (j + 2), hipMemcpyDeviceToHost,
-                                         h->stream));
                 HIPCHK(h, hipStreamSynchronize(h->stream));
+                std::copy(hcol, hcol + j + 2, hc.begin());
                 const double wn = std::sqrt(hc[j + 1]);
-                for (int i = 0; i <= j; i++) Hc(i, j) = hc[i] * nrm[i] / sigma;
-                Hc(j + 1, j) = wn / sigma;
+                for (int i = 0; i <= j; i++) Hc(i, j) = hc[i] * nrm[i] / nrm[j];
+                Hc(j + 1, j) = wn / nrm[j];
                 if (!std::isfinite(wn)) { rc = STZMG_ERR_NONFINITE; break; }
                 nrm[j + 1] = wn;
-                isq[j + 1] = wn > 0 ? 1.0 / (wn * wn) : 0.0;
+                isq.v[j + 1] = wn > 0 ? 1.0 / (wn * wn) : 0.0;
                 for (int i = 0; i < j; i++) {
                     const double a = Hc(i, j), b = Hc(i + 1, j);
                     Hc(i, j) = cs[i] * a + sn[i] * b;
@@ -1949,10 +1950,10 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
                 for (int k2 = i + 1; k2 < nj; k2++) t -= Hc(i, k2) * y[k2];
                 y[i] = t / Hc(i, i);
             }
-            for (int i = 0; i < nj; i++) hc[i] = y[i] / sigma;
-            HIPCHK(h, hipMemcpyAsync(h->kdev, hc.data(), sizeof(double) * nj, hipMemcpyHostToDevice, h->stream));
+            KrylovVals yv{};
+            for (int i = 0; i < nj; i++) yv.v[i] = y[i] / nrm[i];
             hipLaunchKernelGGL(k_xupdate<float>, dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, L.x64, (const float *)h->kZ,
-                               (const double *)h->kdev, nj, n3);
+                               yv, nj, n3);
             LAUNCHCHK(h);
             s.outer++;
             if ((rc = norms64(h, 0, v))) return rc;
@@ -1987,7 +1988,7 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
         const unsigned nb3 = nblk(n3);
         while (rc == 0 && s.res > target && beta > 0) {
             hipLaunchKernelGGL((k_scale<double, double>), dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, h->kV,
-                               (const double *)L.t64, 1.0 / beta, n3);
+                               (const double *)L.t64, 1.0 / beta, n3, (double *)nullptr);
             std::fill(g.begin(), g.end(), 0.0);
             g[0] = beta;
             int nj = 0;
@@ -2005,22 +2006,21 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
                 launch_apply<double>(h, L, (const double *)L.x64, w, zj);
                 launch_mdot_n<1>(h->stream, (const double *)w, (const double *)h->kV, j + 1, n3, h->kpart);
                 hipLaunchKernelGGL(k_reduce_cols, dim3(j + 1), dim3(kThreads), 0, h->stream,
-                                   (const double *)h->kpart, kDotBlocks, j + 1, h->kdev, (const double *)nullptr);
+                                   (const double *)h->kpart, kDotBlocks, j + 1, h->kdev, hcol, 0, KrylovVals{});
                 launch_maxpy_n<1>(h->stream, w, (const double *)h->kV, (const double *)h->kdev, j + 1, n3,
                                   h->kpart);
                 hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(kThreads), 0, h->stream, (const double *)h->kpart,
-                                   kDotBlocks, 1, h->kdev + (j + 1), (const double *)nullptr);
+                                   kDotBlocks, 1, (double *)nullptr, hcol + (j + 1), 0, KrylovVals{});
                 LAUNCHCHK(h);
-                HIPCHK(h, hipMemcpyAsync(hc.data(), h->kdev, sizeof(double) * (j + 2), hipMemcpyDeviceToHost,
-                                         h->stream));
                 HIPCHK(h, hipStreamSynchronize(h->stream));
+                std::copy(hcol, hcol + j + 2, hc.begin());
                 const double wn = std::sqrt(hc[j + 1]);
                 for (int i = 0; i <= j; i++) Hc(i, j) = hc[i];
                 Hc(j + 1, j) = wn;
                 if (!std::isfinite(wn)) { rc = STZMG_ERR_NONFINITE; break; }
                 if (wn > 0)
                     hipLaunchKernelGGL((k_scale<double, double>), dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, w,
-                                       (const double *)w, 1.0 / wn, n3);
+                                       (const double *)w, 1.0 / wn, n3, (double *)nullptr);
                 for (int i = 0; i < j; i++) {
                     const double a = Hc(i, j), b = Hc(i + 1, j);
                     Hc(i, j) = cs[i] * a + sn[i] * b;
@@ -2042,9 +2042,10 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
                 for (int k2 = i + 1; k2 < nj; k2++) t -= Hc(i, k2) * y[k2];
                 y[i] = t / Hc(i, i);
             }
-            HIPCHK(h, hipMemcpyAsync(h->kdev, y.data(), sizeof(double) * nj, hipMemcpyHostToDevice, h->stream));
+            KrylovVals yv{};
+            std::copy(y.begin(), y.begin() + nj, yv.v);
             hipLaunchKernelGGL(k_xupdate<double>, dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, h->kX64,
-                               (const double *)h->kZ64, (const double *)h->kdev, nj, n3);
+                               (const double *)h->kZ64, yv, nj, n3);
             LAUNCHCHK(h);
             s.outer++;
             if ((rc = norms64_of(h, 0, h->kX64, h->kB64, v))) return rc;
