@@ -36,6 +36,7 @@
 // transcendental function enters.
 #pragma clang fp contract(off)
 
+#include "stz_advect.hpp"
 #include "stz_internal.hpp"
 
 using namespace stz;
@@ -48,36 +49,6 @@ struct Dyn {
     double rho, kappa, U;
     double ax, ay, az, Lx, Ly, Lz;
 };
-
-// Velocity component at vertex (i, j, k) with the wall ghosts of the
-// reference's grid: k = -1, -2 extrapolated from planes 0, 1; k = Nz + 1 from
-// the top plate and plane Nz - 1.
-__device__ __forceinline__ double vel_g(const double *__restrict__ u, const Grid &g, int i, int j, int k) {
-    if (g.pz || (k >= 0 && k <= g.Nz)) return vertv(u, g, i, j, k);
-    if (k < 0) {
-        const double a = vertv(u, g, i, j, 0), b = vertv(u, g, i, j, 1);
-        const double m1 = (a + a) - b;
-        return k == -1 ? m1 : (m1 + m1) - a;
-    }
-    const double a = vertv(u, g, i, j, g.Nz), b = vertv(u, g, i, j, g.Nz - 1);
-    return 2 * a - b;
-}
-
-// Reference-map component q at vertex (i, j, k): periodic images shifted by
-// the domain length, zero beyond a wall.
-__device__ __forceinline__ double xi_g(const double *__restrict__ xi, const Grid &g, const Dyn &D, int q, int i,
-                                       int j, int k) {
-    double off = 0;
-    if (q == 0) off = i >= g.Nx ? D.Lx : (i < 0 ? -D.Lx : 0.0);
-    if (q == 1) off = j >= g.Ny ? D.Ly : (j < 0 ? -D.Ly : 0.0);
-    if (g.pz) {
-        if (q == 2) off = k >= g.Nz ? D.Lz : (k < 0 ? -D.Lz : 0.0);
-    } else if (k < 0 || k > g.Nz) {
-        return 0.0;
-    }
-    const double v = vertv(xi + (long)q * g.Nv, g, i, j, k);
-    return off == 0.0 ? v : v + off;
-}
 
 static __global__ __launch_bounds__(kT) void k_direct_plastic(Grid g, Mat M, double dt,
                                                               const double *__restrict__ sig,
@@ -103,204 +74,400 @@ static __global__ __launch_bounds__(kT) void k_direct_plastic(Grid g, Mat M, dou
     dpl_new[c] = D;
 }
 
-static __global__ __launch_bounds__(kT) void k_direct_cell(Grid g, Mat M, double dt, const double *__restrict__ vel,
-                                                           const double *__restrict__ sig,
-                                                           const double *__restrict__ chi,
-                                                           const double *__restrict__ adapt,
-                                                           const double *__restrict__ dchi,
-                                                           const double *__restrict__ dnew,
-                                                           const double *__restrict__ dold,
-                                                           double *__restrict__ sig_out, double *__restrict__ chi_out,
-                                                           BrickGrid B) {
-    int i, j, k;
-    if (!brick_point(B, g.Nx, g.Ny, i, j, k)) return;
-    const long c = i + (long)g.Nx * (j + (long)g.Ny * k);
-    const Stencil5 S = stencil5(g, i, j, k, g.Nz);
-    // away from the walls (uniform over a brick tile, which is one plane)
-    const bool zin = g.pz || (k >= 2 && k <= g.Nz - 3);
-    double G[3][3], v[3];
-    vel_grad_o(vel, g, c, S.ox[3], S.oy[3], S.oz[3], G, v);
-    const double dtlamb = dt * M.lamb, twomudt = 2 * M.mu * dt, dtmu = dt * M.mu;
-    const double hx = g.dx / dt, hy = g.dy / dt, hz = g.dz / dt;
-    double ug[7];
+// Stress and chi of every cell, marching a tile of kAX x kAY cells through a
+// chunk of z planes with the window of k_advect_march (stz_advect.hpp: the
+// seven fields of a plane with a halo of two in LDS, a column's planes
+// k - 2 .. k + 2 in registers, two vertex planes in LDS).  One thread per cell
+// reading its 13-point stencils through the caches waited on some 130 loads
+// at three waves per SIMD: 192 x 192 x 96 cells took 486 us, this form 275 us
+// (0.6 GB of compulsory traffic, about 100 us).  What is left is the wait for
+// a plane's loads between two barriers at two workgroups per CU (242
+// registers; bounded to three it spills 124).
+template <bool PZ>
+static __global__ __launch_bounds__(kT) void k_direct_cell(
+    Grid g, Mat M, double dt, AdvTiles T, const double *__restrict__ vel, const double *__restrict__ sig,
+    const double *__restrict__ chi, const double *__restrict__ adapt, const double *__restrict__ dchi,
+    const double *__restrict__ dnew, const double *__restrict__ dold, double *__restrict__ sig_out,
+    double *__restrict__ chi_out) {
+    constexpr int NF = 7;
+    __shared__ double sc[NF][kSY * kSX];
+    __shared__ double sv[2][3][kVY * kVX];
+
+    const long Lb = xcd_block();
+    const int tx = (int)(Lb % T.ntx), ty = (int)((Lb / T.ntx) % T.nty), zc = (int)(Lb / ((long)T.ntx * T.nty));
+    const int k0 = zc * T.kchunk;
+    if (k0 >= g.Nz) return;
+    const int k1 = k0 + T.kchunk < g.Nz ? k0 + T.kchunk : g.Nz;
+    const int i0 = tx * kAX, j0 = ty * kAY;
+    const int tid = threadIdx.x, lx = tid % kAX, ly = tid / kAX;
+    const int i = i0 + lx, j = j0 + ly;
+    const bool act = i < g.Nx && j < g.Ny;
+    const int nx = g.Nx, ny = g.Ny, nz = g.Nz;
+    const int nxy = nx * ny;
+    const int col = wrapm(i, nx) + nx * wrapm(j, ny);  // load position of this lane
+    const long nc = g.Nc, nv = g.Nv;  // component strides (cell and vertex indices fit in int)
+
+    // The positions a lane stages are those of every plane: formed once.
+    static_assert(kHalo <= 2 * kT && kVX * kVY <= 2 * kT, "two positions per lane");
+    int hp[2], hs[2], vp[2];
 #pragma unroll
-    for (int q = 0; q < 7; q++) {
-        const double *f = q < 6 ? sig + q * g.Nc : chi;
-        const double *fc = f + c;
-        const double f0 = fc[0];
-        const double ddx = eno2(hx, v[0], fc[S.ox[4]], fc[S.ox[3]], f0, fc[S.ox[1]], fc[S.ox[0]]);
-        const double ddy = eno2(hy, v[1], fc[S.oy[4]], fc[S.oy[3]], f0, fc[S.oy[1]], fc[S.oy[0]]);
-        double z2p, z1p, z1m, z2m;
-        if (zin) {
-            z2p = fc[S.oz[4]];
-            z1p = fc[S.oz[3]];
-            z1m = fc[S.oz[1]];
-            z2m = fc[S.oz[0]];
-        } else {
-            z2p = cellv(f, g, i, j, k + 2);
-            z1p = cellv(f, g, i, j, k + 1);
-            z1m = cellv(f, g, i, j, k - 1);
-            z2m = cellv(f, g, i, j, k - 2);
+    for (int e = 0; e < 2; e++) {
+        const int h = tid + e * kT;
+        int sx, sy;
+        halo_pos(h < kHalo ? h : 0, sx, sy);
+        hp[e] = wrapm(i0 + sx - 2, nx) + nx * wrapm(j0 + sy - 2, ny);
+        hs[e] = sy * kSX + sx;
+        const int vy = h / kVX, vx = h - vy * kVX;
+        vp[e] = wrapm(i0 + vx, nx) + nx * wrapm(j0 + vy, ny);
+    }
+    auto stage_vertices = [&](int kv) {
+        const int kw = PZ ? wrapc(kv, nz) : kv;
+        double(*dst)[kVY * kVX] = sv[kv & 1];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const int h = tid + e * kT;
+            if (h < kVX * kVY) {
+                const int q = vp[e] + nxy * kw;
+#pragma unroll
+                for (int d = 0; d < 3; d++) dst[d][h] = vel[d * nv + q];
+            }
         }
-        const double ddz = eno2(hz, v[2], z2p, z1p, f0, z1m, z2m);
-        ug[q] = v[0] * ddx + v[1] * ddy + v[2] * ddz;
+    };
+    // field q (0..5 stress components, 6 chi) at offset p
+    auto F = [&](int q, int p) -> double { return q < 6 ? sig[q * nc + p] : chi[p]; };
+
+    // z window of this thread's column: w[q][s] holds plane k - 2 + s.
+    // Across a wall the ghost planes follow the reference's extrapolation
+    // f(-1) = 2 f(0) - f(1), f(-2) = 2 f(-1) - f(0) and its mirror at the
+    // top, each formed from the two planes next to it in the window.
+    double w[NF][5];
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const int kk = k0 - 2 + s;
+        if (PZ || (kk >= 0 && kk < nz)) {
+            const int p = col + nxy * (PZ ? wrapc(kk, nz) : kk);
+#pragma unroll
+            for (int q = 0; q < NF; q++) w[q][s] = F(q, p);
+        }
     }
-    const double s11 = sig[c], s12 = sig[g.Nc + c], s13 = sig[2 * g.Nc + c];
-    const double s22 = sig[3 * g.Nc + c], s23 = sig[4 * g.Nc + c], s33 = sig[5 * g.Nc + c];
-    const double du_dx = G[0][0], du_dy = G[0][1], du_dz = G[0][2];
-    const double dv_dx = G[1][0], dv_dy = G[1][1], dv_dz = G[1][2];
-    const double dw_dx = G[2][0], dw_dy = G[2][1], dw_dz = G[2][2];
-    const double d_trace = (du_dx + dv_dy + dw_dz);
-    const double t11 = s11 * (du_dx - dv_dy - dw_dz) + 2 * s13 * du_dz + 2 * s12 * du_dy;
-    const double t12 = s23 * du_dz + s13 * dv_dz - s12 * dw_dz + s22 * du_dy + s11 * dv_dx;
-    const double t13 = s33 * du_dz + s11 * dw_dx + s23 * du_dy + s12 * dw_dy - s13 * dv_dy;
-    const double t22 = 2 * s23 * dv_dz + s22 * (dv_dy - du_dx - dw_dz) + 2 * s12 * dv_dx;
-    const double t23 = s33 * dv_dz + s22 * dw_dy + s13 * dv_dx - s23 * du_dx + s12 * dw_dx;
-    const double t33 = s33 * (dw_dz - dv_dy - du_dx) + 2 * s23 * dw_dy + 2 * s13 * dw_dx;
-    double cs11 = dtlamb * d_trace + twomudt * du_dx - ug[0] + dt * t11;
-    double cs22 = dtlamb * d_trace + twomudt * dv_dy - ug[3] + dt * t22;
-    double cs33 = dtlamb * d_trace + twomudt * dw_dz - ug[5] + dt * t33;
-    double cs12 = dtmu * (du_dy + dv_dx) - ug[1] + dt * t12;
-    double cs13 = dtmu * (du_dz + dw_dx) - ug[2] + dt * t13;
-    double cs23 = dtmu * (dv_dz + dw_dy) - ug[4] + dt * t23;
-    const double a = adapt[c];
-    if (a != 0.0) {
-        const double sig_trace = s11 + s22 + s33, third = 1. / 3.;
-        cs11 -= a * (s11 - third * sig_trace);
-        cs12 -= a * (s12);
-        cs13 -= a * (s13);
-        cs22 -= a * (s22 - third * sig_trace);
-        cs23 -= a * (s23);
-        cs33 -= a * (s33 - third * sig_trace);
+    if (!PZ) {
+        if (k0 + 1 >= nz) {
+#pragma unroll
+            for (int q = 0; q < NF; q++) w[q][3] = (w[q][2] + w[q][2]) - w[q][1];
+        }
+#pragma unroll
+        for (int s = 1; s >= 0; s--)
+            if (k0 - 2 + s < 0) {
+#pragma unroll
+                for (int q = 0; q < NF; q++) w[q][s] = (w[q][s + 1] + w[q][s + 1]) - w[q][s + 2];
+            }
     }
-    sig_out[c] = s11 + cs11;
-    sig_out[g.Nc + c] = s12 + cs12;
-    sig_out[2 * g.Nc + c] = s13 + cs13;
-    sig_out[3 * g.Nc + c] = s22 + cs22;
-    sig_out[4 * g.Nc + c] = s23 + cs23;
-    sig_out[5 * g.Nc + c] = s33 + cs33;
-    // chi diffusion (chi_diffusion, src/shear_sim_3d.cpp:1217-1237)
-    const double Dc = dnew[c];
-    const double Dxm = i > 0 ? dnew[c - 1] : dold[c + S.ox[1]];
-    const double Dxp = dold[c + S.ox[3]];
-    const double Dym = j > 0 ? dnew[c - g.Nx] : dold[c + S.oy[1]];
-    const double Dyp = dold[c + S.oy[3]];
-    double Dzm, Dzp;
-    if (g.pz) {
-        Dzm = k > 0 ? dnew[c - (long)g.Nx * g.Ny] : dold[c + S.oz[1]];
-        Dzp = dold[c + S.oz[3]];
-    } else {
-        Dzm = k > 0 ? dnew[c - (long)g.Nx * g.Ny] : 0.0;
-        Dzp = k < g.Nz - 1 ? dold[c + (long)g.Nx * g.Ny] : 0.0;
+    stage_vertices(k0);
+
+    const double hx = g.dx / dt, hy = g.dy / dt, hz = g.dz / dt;
+    const int me = (ly + 2) * kSX + lx + 2;
+    for (int k = k0; k < k1; k++) {
+        if (PZ || k + 2 < nz) {
+            const int p = col + nxy * (PZ ? wrapc(k + 2, nz) : k + 2);
+#pragma unroll
+            for (int q = 0; q < NF; q++) w[q][4] = F(q, p);
+        } else {
+#pragma unroll
+            for (int q = 0; q < NF; q++) w[q][4] = (w[q][3] + w[q][3]) - w[q][2];
+        }
+        __syncthreads();  // the previous plane's LDS reads are done
+#pragma unroll
+        for (int q = 0; q < NF; q++) sc[q][me] = w[q][2];
+#pragma unroll
+        for (int e = 0; e < 2; e++)
+            if (tid + e * kT < kHalo) {
+                const int p = hp[e] + nxy * k;
+#pragma unroll
+                for (int q = 0; q < NF; q++) sc[q][hs[e]] = F(q, p);
+            }
+        stage_vertices(k + 1);
+        __syncthreads();
+
+        if (act) {
+            const int c = i + nx * j + nxy * k;
+            auto S = [&](int q, int dx, int dy) -> double { return sc[q][me + dy * kSX + dx]; };
+            // vertex d of (i + a, j + b, k + e)
+            auto V = [&](int d, int a, int b, int e) -> double {
+                return sv[(k + e) & 1][d][(ly + b) * kVX + lx + a];
+            };
+            // velocity gradient and cell velocity (vel_grad_o)
+            double G[3][3], v[3];
+            {
+                const double gx = .25 * (1.0 / g.dx), gy = .25 * (1.0 / g.dy), gz = .25 * (1.0 / g.dz);
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    const double u000 = V(q, 0, 0, 0), u100 = V(q, 1, 0, 0);
+                    const double u010 = V(q, 0, 1, 0), u110 = V(q, 1, 1, 0);
+                    const double u001 = V(q, 0, 0, 1), u101 = V(q, 1, 0, 1);
+                    const double u011 = V(q, 0, 1, 1), u111 = V(q, 1, 1, 1);
+                    G[q][0] = gx * (u100 - u000 + u110 - u010 + u101 - u001 + u111 - u011);
+                    G[q][1] = gy * (u010 - u000 + u110 - u100 + u011 - u001 + u111 - u101);
+                    G[q][2] = gz * (u001 - u000 + u101 - u100 + u011 - u010 + u111 - u110);
+                    v[q] = 0.125 * (u000 + u100 + u001 + u101 + u010 + u110 + u011 + u111);
+                }
+            }
+            const double dtlamb = dt * M.lamb, twomudt = 2 * M.mu * dt, dtmu = dt * M.mu;
+            double ug[7];
+#pragma unroll
+            for (int q = 0; q < 7; q++) {
+                const double f0 = S(q, 0, 0);
+                const double ddx = eno2(hx, v[0], S(q, 2, 0), S(q, 1, 0), f0, S(q, -1, 0), S(q, -2, 0));
+                const double ddy = eno2(hy, v[1], S(q, 0, 2), S(q, 0, 1), f0, S(q, 0, -1), S(q, 0, -2));
+                const double ddz = eno2(hz, v[2], w[q][4], w[q][3], f0, w[q][1], w[q][0]);
+                ug[q] = v[0] * ddx + v[1] * ddy + v[2] * ddz;
+            }
+            const double s11 = S(0, 0, 0), s12 = S(1, 0, 0), s13 = S(2, 0, 0);
+            const double s22 = S(3, 0, 0), s23 = S(4, 0, 0), s33 = S(5, 0, 0);
+            const double du_dx = G[0][0], du_dy = G[0][1], du_dz = G[0][2];
+            const double dv_dx = G[1][0], dv_dy = G[1][1], dv_dz = G[1][2];
+            const double dw_dx = G[2][0], dw_dy = G[2][1], dw_dz = G[2][2];
+            const double d_trace = (du_dx + dv_dy + dw_dz);
+            const double t11 = s11 * (du_dx - dv_dy - dw_dz) + 2 * s13 * du_dz + 2 * s12 * du_dy;
+            const double t12 = s23 * du_dz + s13 * dv_dz - s12 * dw_dz + s22 * du_dy + s11 * dv_dx;
+            const double t13 = s33 * du_dz + s11 * dw_dx + s23 * du_dy + s12 * dw_dy - s13 * dv_dy;
+            const double t22 = 2 * s23 * dv_dz + s22 * (dv_dy - du_dx - dw_dz) + 2 * s12 * dv_dx;
+            const double t23 = s33 * dv_dz + s22 * dw_dy + s13 * dv_dx - s23 * du_dx + s12 * dw_dx;
+            const double t33 = s33 * (dw_dz - dv_dy - du_dx) + 2 * s23 * dw_dy + 2 * s13 * dw_dx;
+            double cs11 = dtlamb * d_trace + twomudt * du_dx - ug[0] + dt * t11;
+            double cs22 = dtlamb * d_trace + twomudt * dv_dy - ug[3] + dt * t22;
+            double cs33 = dtlamb * d_trace + twomudt * dw_dz - ug[5] + dt * t33;
+            double cs12 = dtmu * (du_dy + dv_dx) - ug[1] + dt * t12;
+            double cs13 = dtmu * (du_dz + dw_dx) - ug[2] + dt * t13;
+            double cs23 = dtmu * (dv_dz + dw_dy) - ug[4] + dt * t23;
+            const double a = adapt[c];
+            if (a != 0.0) {
+                const double sig_trace = s11 + s22 + s33, third = 1. / 3.;
+                cs11 -= a * (s11 - third * sig_trace);
+                cs12 -= a * (s12);
+                cs13 -= a * (s13);
+                cs22 -= a * (s22 - third * sig_trace);
+                cs23 -= a * (s23);
+                cs33 -= a * (s33 - third * sig_trace);
+            }
+            sig_out[c] = s11 + cs11;
+            sig_out[g.Nc + c] = s12 + cs12;
+            sig_out[2 * g.Nc + c] = s13 + cs13;
+            sig_out[3 * g.Nc + c] = s22 + cs22;
+            sig_out[4 * g.Nc + c] = s23 + cs23;
+            sig_out[5 * g.Nc + c] = s33 + cs33;
+            // chi diffusion (chi_diffusion, src/shear_sim_3d.cpp:1217-1237)
+            const double Dc = dnew[c];
+            const double Dxm = i > 0 ? dnew[c - 1] : dold[c + (nx - 1)];
+            const double Dxp = dold[c + (i + 1 < nx ? 1 : 1 - nx)];
+            const double Dym = j > 0 ? dnew[c - nx] : dold[c + (ny - 1) * nx];
+            const double Dyp = dold[c + (j + 1 < ny ? nx : -(ny - 1) * nx)];
+            double Dzm, Dzp;
+            if (PZ) {
+                Dzm = k > 0 ? dnew[c - nxy] : dold[c + (nz - 1) * nxy];
+                Dzp = dold[c + (k + 1 < nz ? nxy : -(nz - 1) * nxy)];
+            } else {
+                Dzm = k > 0 ? dnew[c - nxy] : 0.0;
+                Dzp = k < nz - 1 ? dold[c + nxy] : 0.0;
+            }
+            const double x0 = S(6, 0, 0);
+            const double xxm = S(6, -1, 0), xxp = S(6, 1, 0);
+            const double xym = S(6, 0, -1), xyp = S(6, 0, 1);
+            const double xzm = w[6][1], xzp = w[6][3];
+            const double ix = 1 / g.dx, iy = 1 / g.dy, iz = 1 / g.dz;
+            const double ddx = .5 * ix * (Dxp - Dxm) * (.5 * ix * (xxp - xxm)) + Dc * (ix * ix * (xxp - 2 * x0 + xxm));
+            const double ddy = .5 * iy * (Dyp - Dym) * (.5 * iy * (xyp - xym)) + Dc * (iy * iy * (xyp - 2 * x0 + xym));
+            const double ddz = .5 * iz * (Dzp - Dzm) * (.5 * iz * (xzp - xzm)) + Dc * (iz * iz * (xzp - 2 * x0 + xzm));
+            const double diff = M.diff_l * M.diff_l * (ddx + ddy + ddz);
+            double cchi = dchi[c];
+            cchi -= ug[6];
+            cchi += dt * diff / M.c0;
+            chi_out[c] = x0 + cchi;
+        }
+#pragma unroll
+        for (int q = 0; q < NF; q++)
+#pragma unroll
+            for (int s = 0; s < 4; s++) w[q][s] = w[q][s + 1];
     }
-    const double *xc = chi + c;
-    const double x0 = xc[0];
-    const double xxm = xc[S.ox[1]], xxp = xc[S.ox[3]];
-    const double xym = xc[S.oy[1]], xyp = xc[S.oy[3]];
-    const double xzm = zin ? xc[S.oz[1]] : cellv(chi, g, i, j, k - 1);
-    const double xzp = zin ? xc[S.oz[3]] : cellv(chi, g, i, j, k + 1);
-    const double ix = 1 / g.dx, iy = 1 / g.dy, iz = 1 / g.dz;
-    const double ddx = .5 * ix * (Dxp - Dxm) * (.5 * ix * (xxp - xxm)) + Dc * (ix * ix * (xxp - 2 * x0 + xxm));
-    const double ddy = .5 * iy * (Dyp - Dym) * (.5 * iy * (xyp - xym)) + Dc * (iy * iy * (xyp - 2 * x0 + xym));
-    const double ddz = .5 * iz * (Dzp - Dzm) * (.5 * iz * (xzp - xzm)) + Dc * (iz * iz * (xzp - 2 * x0 + xzm));
-    const double diff = M.diff_l * M.diff_l * (ddx + ddy + ddz);
-    double cchi = dchi[c];
-    cchi -= ug[6];
-    cchi += dt * diff / M.c0;
-    chi_out[c] = x0 + cchi;
 }
 
-static __global__ __launch_bounds__(kT) void k_direct_vertex(Grid g, Dyn D, double dt, const double *__restrict__ vel,
+// Velocity and reference map of every vertex, marching like k_direct_cell: the
+// six fields of a plane with a halo of two in LDS, a column's planes
+// k - 2 .. k + 2 in registers, the stress of cell planes k - 1 and k (one more
+// cell at -x and -y) in LDS.  One thread per vertex took 514 us at
+// 192 x 192 x 96 cells, this form 236 us; bound as k_direct_cell is.  The wall
+// ghosts of the velocity are extrapolated from the two planes next to them
+// (2 f(0) - f(1) at k = -1, its mirror at Nz + 1); the reference map is zero
+// there and shifted by the domain length at the periodic images of a
+// component's own axis.
+template <bool PZ>
+static __global__ __launch_bounds__(kT) void k_direct_vertex(Grid g, Dyn D, double dt, AdvTiles T,
+                                                             const double *__restrict__ vel,
                                                              const double *__restrict__ sig,
                                                              const double *__restrict__ xi,
                                                              double *__restrict__ vel_out,
-                                                             double *__restrict__ xi_out, BrickGrid B) {
-    int i, j, k;
-    if (!brick_point(B, g.Nx, g.Ny, i, j, k)) return;
-    const long p = i + (long)g.Nx * (j + (long)g.Ny * k);
-    if (k == 0 || k >= g.Nz) {
-        // the plane zz = 0 and the top plate are not updated here
-#pragma unroll
-        for (int q = 0; q < 3; q++) {
-            vel_out[q * g.Nv + p] = vel[q * g.Nv + p];
-            xi_out[q * g.Nv + p] = xi[q * g.Nv + p];
+                                                             double *__restrict__ xi_out) {
+    constexpr int NF = 6;
+    __shared__ double sc[NF][kSY * kSX];
+    __shared__ double st[2][6][kVY * kVX];
+
+    const long Lb = xcd_block();
+    const int tx = (int)(Lb % T.ntx), ty = (int)((Lb / T.ntx) % T.nty), zc = (int)(Lb / ((long)T.ntx * T.nty));
+    const int nx = g.Nx, ny = g.Ny, nz = g.Nz, nzv = g.Nzv;
+    const int k0 = zc * T.kchunk;
+    if (k0 >= nzv) return;
+    const int k1 = k0 + T.kchunk < nzv ? k0 + T.kchunk : nzv;
+    const int i0 = tx * kAX, j0 = ty * kAY;
+    const int tid = threadIdx.x, lx = tid % kAX, ly = tid / kAX;
+    const int i = i0 + lx, j = j0 + ly;
+    const bool act = i < nx && j < ny;
+    const int nxy = nx * ny;
+    const int col = wrapm(i, nx) + nx * wrapm(j, ny);  // load position of this lane
+    const long nc = g.Nc, nv = g.Nv;  // component strides (cell and vertex indices fit in int)
+
+    // fields 0..2 velocity, 3..5 reference map at offset p; (a, b) is the
+    // position in the plane, whose periodic images shift the map
+    auto F = [&](int q, int p) -> double { return q < 3 ? vel[q * nv + p] : xi[(q - 3) * nv + p]; };
+    auto shift = [](double v, int a, int n, double len) {
+        return a >= n ? v + len : (a < 0 ? v - len : v);
+    };
+    auto image = [&](int q, double v, int a, int b) {
+        return q == 3 ? shift(v, a, nx, D.Lx) : (q == 4 ? shift(v, b, ny, D.Ly) : v);
+    };
+    // plane kk of field q in this lane's column
+    auto Z = [&](int q, int kk) -> double {
+        if (PZ) {
+            const double v = F(q, col + nxy * wrapc(kk, nz));
+            return q == 5 ? shift(v, kk, nz, D.Lz) : v;
         }
-        return;
+        return F(q, col + nxy * kk);
+    };
+    int hp[2], hs[2], vp[2];  // the positions a lane stages of every plane
+    int ha[2], hb[2];         // and their place before wrapping
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+        const int h = tid + e * kT;
+        int sx, sy;
+        halo_pos(h < kHalo ? h : 0, sx, sy);
+        const int a = i0 + sx - 2, b = j0 + sy - 2;
+        hp[e] = wrapm(a, nx) + nx * wrapm(b, ny);
+        hs[e] = sy * kSX + sx;
+        ha[e] = a;
+        hb[e] = b;
+        const int vy = h / kVX, vx = h - vy * kVX;
+        vp[e] = wrapm(i0 + vx - 1, nx) + nx * wrapm(j0 + vy - 1, ny);
     }
+    auto stage_stress = [&](int kc) {
+        double(*dst)[kVY * kVX] = st[kc & 1];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const int h = tid + e * kT;
+            if (h < kVX * kVY) {
+                const int p = vp[e] + nxy * kc;
+#pragma unroll
+                for (int q = 0; q < 6; q++) dst[q][h] = sig[q * nc + p];
+            }
+        }
+    };
+
+    double w[NF][5];
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const int kk = k0 - 2 + s;
+        if (PZ || (kk >= 0 && kk < nzv)) {
+#pragma unroll
+            for (int q = 0; q < NF; q++) w[q][s] = Z(q, kk);
+        } else {
+#pragma unroll
+            for (int q = 0; q < NF; q++) w[q][s] = 0.0;
+        }
+    }
+    if (k0 > 0) stage_stress(k0 - 1);
+
     const double dx_inv = 1. / g.dx, dy_inv = 1. / g.dy, dz_inv = 1. / g.dz;
     const double dx_inv_sq = dx_inv * dx_inv, dy_inv_sq = dy_inv * dy_inv, dz_inv_sq = dz_inv * dz_inv;
     const double rho_inv = 1. / D.rho;
     const double dtrho_inv = dt * rho_inv, dtkaprho_inv = D.kappa * dtrho_inv;
     const double dxdt = g.dx / dt, dydt = g.dy / dt, dzdt = g.dz / dt;
-    // backward staggered stress derivatives (calculate_first_order_stresses,
-    // src/shear_sim_3d.cpp:971-987): cells (i-1..i, j-1..j, k-1..k)
-    // (0 < k < Nz here, so the cell planes k - 1 and k exist and the cell
-    // index of (i, j, k) is p)
-    const Stencil5 S = stencil5(g, i, j, k, g.Nzv);
-    const bool zin = g.pz || (k >= 2 && k <= g.Nzv - 3);  // no wall ghost in the z stencils
-    const int mx = S.ox[1], my = S.oy[1], mz = S.oz[1];
-    const long c000 = p, c100 = p + mx, c010 = p + my, c110 = p + mx + my, c001 = p + mz, c101 = p + mx + mz,
-               c011 = p + my + mz, c111 = p + mx + my + mz;
-    auto DX = [&](const double *a) {
-        return .25 * dx_inv * (a[c000] - a[c100] + a[c010] - a[c110] + a[c001] - a[c101] + a[c011] - a[c111]);
-    };
-    auto DY = [&](const double *a) {
-        return .25 * dy_inv * (a[c000] - a[c010] + a[c100] - a[c110] + a[c001] - a[c011] + a[c101] - a[c111]);
-    };
-    auto DZ = [&](const double *a) {
-        return .25 * dz_inv * (a[c000] - a[c001] + a[c100] - a[c101] + a[c010] - a[c011] + a[c110] - a[c111]);
-    };
-    const double *S11 = sig, *S12 = sig + g.Nc, *S13 = sig + 2 * g.Nc, *S22 = sig + 3 * g.Nc, *S23 = sig + 4 * g.Nc,
-                 *S33 = sig + 5 * g.Nc;
-    const double div[3] = {DX(S11) + DY(S12) + DZ(S13), DX(S12) + DY(S22) + DZ(S23), DX(S13) + DY(S23) + DZ(S33)};
-    const double u = vel[p], v = vel[g.Nv + p], w = vel[2 * g.Nv + p];
+    const int me = (ly + 2) * kSX + lx + 2, mv = (ly + 1) * kVX + lx + 1;
+    for (int k = k0; k < k1; k++) {
+        if (PZ || k + 2 < nzv) {
 #pragma unroll
-    for (int q = 0; q < 3; q++) {
-        const double *f = vel + q * g.Nv;
-        const double *fp = f + p;
-        const double f0 = fp[0];
-        double z2p, z1p, z1m, z2m;
-        if (zin) {
-            z2p = fp[S.oz[4]];
-            z1p = fp[S.oz[3]];
-            z1m = fp[S.oz[1]];
-            z2m = fp[S.oz[0]];
+            for (int q = 0; q < NF; q++) w[q][4] = Z(q, k + 2);
         } else {
-            z2p = vel_g(f, g, i, j, k + 2);
-            z1p = vel_g(f, g, i, j, k + 1);
-            z1m = vel_g(f, g, i, j, k - 1);
-            z2m = vel_g(f, g, i, j, k - 2);
+            // only plane Nz + 1, seen from Nz - 1, is used
+#pragma unroll
+            for (int q = 0; q < NF; q++) w[q][4] = q < 3 ? (w[q][3] + w[q][3]) - w[q][2] : 0.0;
         }
-        const double gsq = dx_inv_sq * (fp[S.ox[3]] - 2 * f0 + fp[S.ox[1]]) +
-                           dy_inv_sq * (fp[S.oy[3]] - 2 * f0 + fp[S.oy[1]]) + dz_inv_sq * (z1p - 2 * f0 + z1m);
-        const double ddx = eno2(dxdt, u, fp[S.ox[4]], fp[S.ox[3]], f0, fp[S.ox[1]], fp[S.ox[0]]);
-        const double ddy = eno2(dydt, v, fp[S.oy[4]], fp[S.oy[3]], f0, fp[S.oy[1]], fp[S.oy[0]]);
-        const double ddz = eno2(dzdt, w, z2p, z1p, f0, z1m, z2m);
-        const double ugq = u * ddx + v * ddy + w * ddz;
-        vel_out[q * g.Nv + p] = f0 + (dtrho_inv * div[q] + dtkaprho_inv * gsq - ugq);
-        // reference map: the periodic image of component q along axis q is
-        // shifted by the domain length, as xi_g does it
-        const double *xp = xi + q * g.Nv + p;
-        const double x0 = xp[0];
-        auto img = [&](const int(&o)[5], int n, int a, double Lq, bool axis) {
-            const double val = xp[o[a]];
-            if (!axis || o[a] == (a - 2) * n) return val;
-            const double off = a > 2 ? Lq : -Lq;
-            return off == 0.0 ? val : val + off;
-        };
-        const int nxy = g.Nx * g.Ny;
-        const double ex = eno2(dxdt, u, img(S.ox, 1, 4, D.Lx, q == 0), img(S.ox, 1, 3, D.Lx, q == 0), x0,
-                               img(S.ox, 1, 1, D.Lx, q == 0), img(S.ox, 1, 0, D.Lx, q == 0));
-        const double ey = eno2(dydt, v, img(S.oy, g.Nx, 4, D.Ly, q == 1), img(S.oy, g.Nx, 3, D.Ly, q == 1), x0,
-                               img(S.oy, g.Nx, 1, D.Ly, q == 1), img(S.oy, g.Nx, 0, D.Ly, q == 1));
-        double ez;
-        if (zin)
-            ez = eno2(dzdt, w, img(S.oz, nxy, 4, D.Lz, q == 2), img(S.oz, nxy, 3, D.Lz, q == 2), x0,
-                      img(S.oz, nxy, 1, D.Lz, q == 2), img(S.oz, nxy, 0, D.Lz, q == 2));
-        else
-            ez = eno2(dzdt, w, xi_g(xi, g, D, q, i, j, k + 2), xi_g(xi, g, D, q, i, j, k + 1), x0,
-                      xi_g(xi, g, D, q, i, j, k - 1), xi_g(xi, g, D, q, i, j, k - 2));
-        xi_out[q * g.Nv + p] = x0 + (0.0 - (u * ex + v * ey + w * ez));
+        if (!PZ && k == 1) {
+#pragma unroll
+            for (int q = 0; q < 3; q++) w[q][0] = (w[q][1] + w[q][1]) - w[q][2];
+        }
+        __syncthreads();  // the previous plane's LDS reads are done
+#pragma unroll
+        for (int q = 0; q < NF; q++) sc[q][me] = image(q, w[q][2], i, j);
+#pragma unroll
+        for (int e = 0; e < 2; e++)
+            if (tid + e * kT < kHalo) {
+                const int p = hp[e] + nxy * k;
+#pragma unroll
+                for (int q = 0; q < NF; q++) sc[q][hs[e]] = image(q, F(q, p), ha[e], hb[e]);
+            }
+        if (k < nz) stage_stress(k);
+        __syncthreads();
+
+        if (act) {
+            const int p = i + nx * j + nxy * k;
+            if (k == 0 || k >= nz) {
+                // the plane zz = 0 and the top plate are not updated here
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    vel_out[q * nv + p] = w[q][2];
+                    xi_out[q * nv + p] = w[3 + q][2];
+                }
+            } else {
+                auto S = [&](int q, int dx, int dy) -> double { return sc[q][me + dy * kSX + dx]; };
+                // backward staggered stress derivatives
+                // (calculate_first_order_stresses,
+                // src/shear_sim_3d.cpp:971-987): cells (i-1..i, j-1..j, k-1..k)
+                const double(*hi)[kVY * kVX] = st[k & 1], (*lo)[kVY * kVX] = st[(k - 1) & 1];
+                auto DX = [&](int q) {
+                    const double *a = hi[q] + mv, *b = lo[q] + mv;
+                    return .25 * dx_inv * (a[0] - a[-1] + a[-kVX] - a[-kVX - 1] + b[0] - b[-1] + b[-kVX] - b[-kVX - 1]);
+                };
+                auto DY = [&](int q) {
+                    const double *a = hi[q] + mv, *b = lo[q] + mv;
+                    return .25 * dy_inv * (a[0] - a[-kVX] + a[-1] - a[-kVX - 1] + b[0] - b[-kVX] + b[-1] - b[-kVX - 1]);
+                };
+                auto DZ = [&](int q) {
+                    const double *a = hi[q] + mv, *b = lo[q] + mv;
+                    return .25 * dz_inv * (a[0] - b[0] + a[-1] - b[-1] + a[-kVX] - b[-kVX] + a[-kVX - 1] - b[-kVX - 1]);
+                };
+                const double div[3] = {DX(0) + DY(1) + DZ(2), DX(1) + DY(3) + DZ(4), DX(2) + DY(4) + DZ(5)};
+                const double u = w[0][2], v = w[1][2], ww = w[2][2];
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    const double f0 = w[q][2], z1p = w[q][3], z1m = w[q][1];
+                    const double xp = S(q, 1, 0), xm = S(q, -1, 0), yp = S(q, 0, 1), ym = S(q, 0, -1);
+                    const double gsq = dx_inv_sq * (xp - 2 * f0 + xm) + dy_inv_sq * (yp - 2 * f0 + ym) +
+                                       dz_inv_sq * (z1p - 2 * f0 + z1m);
+                    const double ddx = eno2(dxdt, u, S(q, 2, 0), xp, f0, xm, S(q, -2, 0));
+                    const double ddy = eno2(dydt, v, S(q, 0, 2), yp, f0, ym, S(q, 0, -2));
+                    const double ddz = eno2(dzdt, ww, w[q][4], z1p, f0, z1m, w[q][0]);
+                    const double ugq = u * ddx + v * ddy + ww * ddz;
+                    vel_out[q * nv + p] = f0 + (dtrho_inv * div[q] + dtkaprho_inv * gsq - ugq);
+                    const int x = 3 + q;
+                    const double x0 = w[x][2];
+                    const double ex = eno2(dxdt, u, S(x, 2, 0), S(x, 1, 0), x0, S(x, -1, 0), S(x, -2, 0));
+                    const double ey = eno2(dydt, v, S(x, 0, 2), S(x, 0, 1), x0, S(x, 0, -1), S(x, 0, -2));
+                    const double ez = eno2(dzdt, ww, w[x][4], w[x][3], x0, w[x][1], w[x][0]);
+                    xi_out[q * nv + p] = x0 + (0.0 - (u * ex + v * ey + ww * ez));
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < NF; q++)
+#pragma unroll
+            for (int s = 0; s < 4; s++) w[q][s] = w[q][s + 1];
     }
 }
 
@@ -395,6 +562,50 @@ Dyn dyn_of(const stz_t s) {
     return Dyn{p.rho, p.kappa, p.U, p.ax, p.ay, p.az, p.bx - p.ax, p.by - p.ay, p.bz - p.az};
 }
 
+// Workgroups of a marching kernel the device keeps resident at once: one
+// round of the launch.
+template <typename F>
+int resident(F *kernel) {
+    int dev = 0, ncu = 0, per = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
+        ncu = 256;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, kT, 0) != hipSuccess || per < 1) per = 1;
+    return ncu * per;
+}
+
+template <bool PZ>
+void launch_cell_z(stz_t s, double dt) {
+    const Grid &g = s->g;
+    int &r = s->direct_resident[PZ ? 1 : 0];
+    if (r <= 0) r = resident(&k_direct_cell<PZ>);
+    const AdvTiles t = adv_tiles(g, r);
+    hipLaunchKernelGGL((k_direct_cell<PZ>), dim3((unsigned)((long)t.ntx * t.nty * t.nzc)), dim3(kT), 0, s->stream, g,
+                       s->M, dt, t, (const double *)s->vel, (const double *)s->sig, (const double *)s->chi,
+                       (const double *)s->adapt, (const double *)s->dchi, (const double *)s->dpl2,
+                       (const double *)s->dpl, s->sig2, s->chi2);
+}
+void launch_cell(stz_t s, double dt) {
+    if (s->g.pz) launch_cell_z<true>(s, dt);
+    else launch_cell_z<false>(s, dt);
+}
+
+template <bool PZ>
+void launch_vertex_z(stz_t s, const Dyn &D, double dt) {
+    Grid g = s->g;
+    int &r = s->direct_resident[PZ ? 3 : 2];
+    if (r <= 0) r = resident(&k_direct_vertex<PZ>);
+    g.Nz = g.Nzv;  // the planes the tiles march through
+    const AdvTiles t = adv_tiles(g, r);
+    hipLaunchKernelGGL((k_direct_vertex<PZ>), dim3((unsigned)((long)t.ntx * t.nty * t.nzc)), dim3(kT), 0, s->stream,
+                       s->g, D, dt, t, (const double *)s->vel, (const double *)s->sig, (const double *)s->xi, s->vel2,
+                       s->xi2);
+}
+void launch_vertex(stz_t s, const Dyn &D, double dt) {
+    if (s->g.pz) launch_vertex_z<true>(s, D, dt);
+    else launch_vertex_z<false>(s, D, dt);
+}
+
 int ensure_ref_map(stz_t s) {
     if (s->xi) return 0;
     const Grid &g = s->g;
@@ -467,19 +678,13 @@ int stz_step_direct(stz_t s, double dt, int nsteps, stz_step_stats *st) {
     if (int rc = ensure_ref_map(s)) return rc;
     const Grid &g = s->g;
     const Dyn D = dyn_of(s);
-    const BrickGrid bc = brick_grid(g.Nx, g.Ny, g.Nz), bv = brick_grid(g.Nx, g.Ny, g.Nzv);
     stz_step_stats S{};
     for (int q = 0; q < nsteps; q++) {
         DHIP(s, hipMemsetAsync(s->counters, 0, sizeof(int) * kCountInts, s->stream));
         hipLaunchKernelGGL(k_direct_plastic, dim3(nbk(g.Nc)), dim3(kT), 0, s->stream, g, s->M, dt,
                            (const double *)s->sig, (const double *)s->chi, s->adapt, s->dchi, s->dpl2, s->counters);
-        hipLaunchKernelGGL(k_direct_cell, dim3(brick_blocks(bc)), dim3(kT), 0, s->stream, g, s->M, dt,
-                           (const double *)s->vel, (const double *)s->sig, (const double *)s->chi,
-                           (const double *)s->adapt, (const double *)s->dchi, (const double *)s->dpl2,
-                           (const double *)s->dpl, s->sig2, s->chi2, bc);
-        hipLaunchKernelGGL(k_direct_vertex, dim3(brick_blocks(bv)), dim3(kT), 0, s->stream, g, D, dt,
-                           (const double *)s->vel, (const double *)s->sig, (const double *)s->xi, s->vel2, s->xi2,
-                           bv);
+        launch_cell(s, dt);
+        launch_vertex(s, D, dt);
         DHIP(s, hipGetLastError());
         std::swap(s->sig, s->sig2);
         std::swap(s->chi, s->chi2);
@@ -537,7 +742,6 @@ int stz_direct_time_kernels(stz_t s, double dt, int reps, double ms[4]) {
     if (int rc = ensure_ref_map(s)) return rc;
     const Grid &g = s->g;
     const Dyn D = dyn_of(s);
-    const BrickGrid bc = brick_grid(g.Nx, g.Ny, g.Nz), bv = brick_grid(g.Nx, g.Ny, g.Nzv);
     hipEvent_t e0, e1;
     DHIP(s, hipEventCreate(&e0));
     DHIP(s, hipEventCreate(&e1));
@@ -550,14 +754,9 @@ int stz_direct_time_kernels(stz_t s, double dt, int reps, double ms[4]) {
                                (const double *)s->sig, (const double *)s->chi, s->adapt, s->dchi, s->dpl2,
                                s->counters);
         else if (which == 1)
-            hipLaunchKernelGGL(k_direct_cell, dim3(brick_blocks(bc)), dim3(kT), 0, s->stream, g, s->M, dt,
-                               (const double *)s->vel, (const double *)s->sig, (const double *)s->chi,
-                               (const double *)s->adapt, (const double *)s->dchi, (const double *)s->dpl2,
-                               (const double *)s->dpl, s->sig2, s->chi2, bc);
+            launch_cell(s, dt);
         else if (which == 2)
-            hipLaunchKernelGGL(k_direct_vertex, dim3(brick_blocks(bv)), dim3(kT), 0, s->stream, g, D, dt,
-                               (const double *)s->vel, (const double *)s->sig, (const double *)s->xi, s->vel2,
-                               s->xi2, bv);
+            launch_vertex(s, D, dt);
         else
             hipLaunchKernelGGL(k_direct_plate, dim3(nbk((long)g.Nx * g.Ny)), dim3(kT), 0, s->stream, g, D, s->t,
                                s->vel, s->xi);

@@ -35,6 +35,7 @@ struct stz_s {
     double user_T[9] = {0}, user_dT[9] = {0};  // stz_set_transform: T(t) = user_T + (t - user_t0) user_dT
     double user_t0 = 0;
     int adv_resident[4] = {0, 0, 0, 0};  // resident workgroups of the k_advect_march variants
+    int direct_resident[4] = {0, 0, 0, 0};  // resident workgroups of the marching direct kernels
     std::string err;
 };
 
