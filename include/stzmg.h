@@ -186,9 +186,10 @@ enum { STZMG_OPT_COARSE_KERNEL = 0, STZMG_OPT_FUSED_SMOOTHER = 1, STZMG_OPT_TILE
        STZMG_OPT_BOTTOM_MAP = 3, STZMG_OPT_CHUNK_CAP = 4, STZMG_OPT_RESTRICT_PLANES = 5,
        STZMG_OPT_CENTRO_GALERKIN = 6 };
 /*   STZMG_OPT_FUSED_SMOOTHER 1 (default): per-plane levels with periodic x, y
- *                            (x and y sizes multiples of 8, more than 1024
- *                            points) sweep with two fused launches (one per z
- *                            parity); 0: eight colour launches per sweep.
+ *                            (x and y sizes even and at least 8, more than
+ *                            1024 points) sweep with two fused launches (one
+ *                            per z parity) or, where small or not in tiles of
+ *                            8, with one; 0: eight colour launches per sweep.
  *   STZMG_OPT_TILED_RESIDUAL 1 (default): on the same levels the residual
  *                            marches tiles through z with planes staged in
  *                            LDS; 0: one thread per point reading its 27
@@ -211,7 +212,8 @@ enum { STZMG_OPT_COARSE_KERNEL = 0, STZMG_OPT_FUSED_SMOOTHER = 1, STZMG_OPT_TILE
  *                            value > 0 caps that count at `value` workgroups,
  *                            so small grids also march several planes per
  *                            workgroup (sweeps unchanged; residual norms may
- *                            differ in the last bits).
+ *                            differ in the last bits).  Levels swept in one
+ *                            launch march no planes and ignore it.
  *   STZMG_OPT_RESTRICT_PLANES 0 (default): coarse planes per restriction
  *                            thread chosen from the grid; value > 0 fixes it
  *                            (results unchanged).
