@@ -260,8 +260,8 @@ constexpr int halo_threads() {
 }
 
 // Grid: (ceil(m / TX), ceil(n / TY), ceil(o / 2)).  PLANE operator, x and y
-// periodic, m and n even and at least 8, o odd (walls) or even and at least
-// 4 (periodic).  pk: rows of march_stride(KEY) values per plane.  zero: x is
+// periodic, m and n even and at least 8, o at least 4, any number (walls) or
+// even (periodic).  Blocks that point across a wall add nothing.  pk: rows of march_stride(KEY) values per plane.  zero: x is
 // zero whatever the buffer holds.  xc (may be null): the sweep starts from
 // x + P xc, the coarse level's correction (dimensions C) added as the window
 // arrives, in interp_point's order -- the correction costs no pass over x and
@@ -386,7 +386,9 @@ __global__ __launch_bounds__((halo_threads<TX, TY>())) __attribute__((amdgpu_wav
     const int hf = (wv / (NW / 4)) & 1;
     const int t0 = tid % (NT / 4);
     const int kA = plane(k0 + 2 * pl);
-    const bool live = pl == 0 || odd;                    // plane k0 + 2 serves plane k0 + 1 only
+    // plane k0 + 2 serves plane k0 + 1 only; above a wall there is none (its
+    // slot of the window stays zero)
+    const bool live = pl == 0 || (odd && (d.pz || k0 + 2 < d.o));
     int cen[2];      // window index of the point in its plane, component 0
     bool own[2];
     T rr[2][3];

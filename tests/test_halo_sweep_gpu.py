@@ -32,7 +32,7 @@ def f32(a):
     return np.asarray(a, dtype=np.float32).astype(np.float64)
 
 
-def planes_of(kind, m, n, o, pz):
+def planes_of(kind, m, n, o, pz, outward=False):
     hx, hy, hz = 1.0 / m, 1.0 / n, 1.0 / o
     st, fix = MG.shear_stencil(1.0, 1.5, hx, hy, hz, 1.0)
     if kind in ("trans", "full"):
@@ -49,7 +49,7 @@ def planes_of(kind, m, n, o, pz):
         planes = np.array(planes).reshape(o, 27, 3, 3)
         planes += 0.02 * np.abs(planes).max() * rng.uniform(-1, 1, planes.shape) * (planes.any(axis=(1, 2, 3)))[
             :, None, None, None]
-        if not pz:
+        if not pz and not outward:
             planes[0, :9] = 0
             planes[-1, 18:] = 0
     return np.ascontiguousarray(planes)
@@ -69,6 +69,38 @@ def test_one_launch_sweep(kind, m, n, o, pz):
     mg = MG.Multigrid(m, n, o, prd, coarsest_total=N)  # this level alone
     mg.setup_matrices_planes(planes)
     orc = O.OracleMG(m, n, o, prd, mode=O.PLANE, coarsest_total=N)
+    orc.set_ops(0, planes)
+    orc.params(smoother=1)
+    mg.setup_fields(x, r)
+    orc.set_fields(0, x, r)
+    mg.gauss_seidel(0, 3)
+    orc.gs(0, 3)
+    assert relerr(mg.x(0), orc.fields(0)[0]) < 1e-12
+    mg.setup_fields(x, r)
+    orc.set_fields(0, f32(x), f32(r))
+    mg.gauss_seidel_fp32(0, 1)
+    orc.gs(0, 1)
+    assert relerr(mg.x(0), orc.fields(0)[0]) < 2e-6
+
+
+@pytest.mark.parametrize("m,n,o", [(20, 28, 4), (16, 16, 10), (20, 28, 6), (12, 10, 18), (8, 16, 12), (64, 64, 16),
+                                   (16, 16, 9)])
+@pytest.mark.parametrize("kind", ["shear", "full", "plain"])
+def test_walls_with_blocks_that_point_outward(kind, m, n, o):
+    """Walls with an even number of planes, whose last pair has no plane above
+    it, and with blocks of the two outermost planes that point across the
+    wall: nothing lies there, so they add nothing.  Such a level is the
+    coarsest one (only odd numbers of walled planes are coarsened).  Rounding
+    as above."""
+    planes = planes_of(kind, m, n, o, 0, outward=True)
+    if kind != "plain":
+        planes[0], planes[-1] = planes[1], planes[1]
+    assert planes.reshape(o, 27, 9)[-1, 18:].any() and planes.reshape(o, 27, 9)[0, :9].any()
+    N = m * n * o
+    x, r = O.det_field(N, 61), O.det_field(N, 62)
+    mg = MG.Multigrid(m, n, o, (1, 1, 0), coarsest_total=N)
+    mg.setup_matrices_planes(planes)
+    orc = O.OracleMG(m, n, o, (1, 1, 0), mode=O.PLANE, coarsest_total=N)
     orc.set_ops(0, planes)
     orc.params(smoother=1)
     mg.setup_fields(x, r)
