@@ -70,12 +70,14 @@ __global__ __launch_bounds__(kThreads) void k_mdot(const TV *__restrict__ w, con
     }
 }
 
-// w -= sum_j coef[j] V_j (j < NV) in FP64, stored as TV (also to copy unless
-// null), then part[b] = block share of |w|^2 (of the stored values).
+// w -= sum_j coef[j] V_j (j < NV) in FP64, stored as TV (also, times the power
+// of two cs, to copy unless null), then part[b] = block share of |w|^2 (of the
+// stored values).
 template <int NV, typename TV = double>
 __global__ __launch_bounds__(kThreads) void k_maxpy_norm(TV *__restrict__ w, const TV *__restrict__ V,
                                                          const double *__restrict__ coef, long n3,
-                                                         double *__restrict__ part, TV *__restrict__ copy) {
+                                                         double *__restrict__ part, TV *__restrict__ copy,
+                                                         TV cs) {
     double c[NV];
 #pragma unroll
     for (int j = 0; j < NV; j++) c[j] = coef[j];
@@ -99,7 +101,7 @@ __global__ __launch_bounds__(kThreads) void k_maxpy_norm(TV *__restrict__ w, con
             for (int j = 0; j < NV; j++) wi -= c[j] * (double)vv[u][j];
             const TV ws = (TV)wi;
             w[i + u * S] = ws;
-            if (copy) copy[i + u * S] = ws;
+            if (copy) copy[i + u * S] = cs * ws;
             acc += (double)ws * (double)ws;
         }
     }
@@ -109,7 +111,7 @@ __global__ __launch_bounds__(kThreads) void k_maxpy_norm(TV *__restrict__ w, con
         for (int j = 0; j < NV; j++) wi -= c[j] * (double)V[(long)j * n3 + i];
         const TV ws = (TV)wi;
         w[i] = ws;
-        if (copy) copy[i] = ws;
+        if (copy) copy[i] = cs * ws;
         acc += (double)ws * (double)ws;
     }
     __shared__ double red[kThreads / 64];
@@ -137,14 +139,14 @@ void launch_mdot_n(hipStream_t st, const TV *w, const TV *V, int nv, long n3, do
 }
 template <int NV, typename TV = double>
 void launch_maxpy_n(hipStream_t st, TV *w, const TV *V, const double *coef, int nv, long n3, double *part,
-                    TV *copy = nullptr) {
+                    TV *copy = nullptr, TV cs = 1) {
     if constexpr (NV <= kKrylovMax + 1) {
         if (nv == NV) {
             hipLaunchKernelGGL((k_maxpy_norm<NV, TV>), dim3(kDotBlocks), dim3(kThreads), 0, st, w, V, coef, n3,
-                               part, copy);
+                               part, copy, cs);
             return;
         }
-        launch_maxpy_n<NV + 1, TV>(st, w, V, coef, nv, n3, part, copy);
+        launch_maxpy_n<NV + 1, TV>(st, w, V, coef, nv, n3, part, copy, cs);
     }
 }
 
@@ -178,11 +180,11 @@ static __global__ __launch_bounds__(kThreads) void k_reduce_cols(const double *_
     }
 }
 
-// dst = a src (in FP64, stored as TD, also to copy unless null; kEW elements
-// per thread, grid nblk_ew(n3)).
+// dst = a src (in FP64, stored as TD, also, times the power of two cs, to copy
+// unless null; kEW elements per thread, grid nblk_ew(n3)).
 template <typename TD = double, typename TS = double>
 __global__ __launch_bounds__(kThreads) void k_scale(TD *__restrict__ dst, const TS *__restrict__ src, double a,
-                                                    long n3, TD *__restrict__ copy = nullptr) {
+                                                    long n3, TD *__restrict__ copy = nullptr, TD cs = 1) {
     const long b0 = (long)blockIdx.x * (kThreads * kEW) + threadIdx.x;
     TS v[kEW];
 #pragma unroll
@@ -194,8 +196,9 @@ __global__ __launch_bounds__(kThreads) void k_scale(TD *__restrict__ dst, const 
     for (int u = 0; u < kEW; u++) {
         const long i = b0 + (long)u * kThreads;
         if (i < n3) {
-            dst[i] = (TD)(a * (double)v[u]);
-            if (copy) copy[i] = (TD)(a * (double)v[u]);
+            const TD t = (TD)(a * (double)v[u]);
+            dst[i] = t;
+            if (copy) copy[i] = cs * t;
         }
     }
 }

@@ -1784,7 +1784,7 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
         const unsigned nb3 = nblk(n3);
         while (rc == 0 && s.res > target && beta > 0) {
             hipLaunchKernelGGL((k_scale<double, double>), dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, h->kV, (const double *)L.t64,
-                               1.0 / beta, n3, (double *)nullptr);
+                               1.0 / beta, n3, (double *)nullptr, 1.0);
             std::fill(g.begin(), g.end(), 0.0);
             g[0] = beta;
             int nj = 0;
@@ -1819,7 +1819,7 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
                 if (!std::isfinite(wn)) { rc = STZMG_ERR_NONFINITE; break; }
                 if (wn > 0)
                     hipLaunchKernelGGL((k_scale<double, double>), dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, w, (const double *)w,
-                                       1.0 / wn, n3, (double *)nullptr);
+                                       1.0 / wn, n3, (double *)nullptr, 1.0);
                 // Givens rotations
                 for (int i = 0; i < j; i++) {
                     const double a = Hc(i, j), b = Hc(i + 1, j);
@@ -1868,13 +1868,16 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
         //
         // Basis vectors are kept unnormalised: u_j = nrm_j v_j.  The
         // reduction of the dot products scales (w, u_i) by 1/nrm_i^2, which
-        // gives the Gram-Schmidt coefficient of u_i directly, and the
-        // preconditioner takes u_j as it is (z_j = M^-1 u_j; nrm_j enters the
-        // Hessenberg column and the update): the pass that forms u_j also
-        // writes it as the V-cycle's right-hand side, so neither a
-        // normalisation nor a defect pass runs (the defect pass took 91 us at
-        // 256^3).  u_j shrinks with the residual only, by at most the few
-        // orders a cycle gains, far from the limits of FP32.
+        // gives the Gram-Schmidt coefficient of u_i directly, and the pass
+        // that forms u_j also writes 2^e_j u_j as the V-cycle's right-hand side
+        // (z_j = M^-1 2^e_j u_j; rho_j = 2^e_j nrm_j enters the Hessenberg
+        // column and the update), so neither a normalisation nor a defect pass
+        // runs (the defect pass took 91 us at 256^3).  2^e_j brings |2^e_j u_j|
+        // to sigma = sqrt(3 N) times what the iteration before gained, whatever
+        // the operator's scale and however far the inner solve goes: entries
+        // near one, where FP32 has most room on both sides for z.  (e_j comes
+        // from the norm before, since u_j is written before its own is known; a
+        // power of two rounds nothing.)
         Level &L = h->lv[0];
         const long n3 = 3 * L.d.N;
         const int m = std::min(std::max(opts->restart, 1), kKrylovMax);
@@ -1887,16 +1890,20 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
         const double inner_rtol = opts->inner_rtol > 0 ? opts->inner_rtol : 1e-4;
         const int inner = opts->inner_cycles > 0 ? opts->inner_cycles : 1;
         if (!std::isfinite(beta)) rc = STZMG_ERR_NONFINITE;
-        std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), g(m + 1), y(m), hc(m + 2), nrm(m + 1);
+        std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), g(m + 1), y(m), hc(m + 2), nrm(m + 1), rho(m + 1);
         auto Hc = [&](int i, int j) -> double & { return H[(size_t)i * m + j]; };
-        const unsigned nb3 = nblk(n3);
+        // power of two nearest v, within FP32
+        auto pow2 = [](double v) { return std::ldexp(1.0, std::min(std::max((int)std::lround(std::log2(v)), -100), 100)); };
+        const double sigma = std::sqrt((double)n3);
         KrylovVals isq{};  // 1/nrm_i^2
         while (rc == 0 && s.res > target && beta > 0) {
+            double e2 = pow2(sigma);
             hipLaunchKernelGGL((k_scale<float, double>), dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, h->kV32,
-                               (const double *)L.t64, 1.0 / beta, n3, L.r32);
+                               (const double *)L.t64, 1.0 / beta, n3, L.r32, (float)e2);
             std::fill(g.begin(), g.end(), 0.0);
             g[0] = beta;
             nrm[0] = 1.0;
+            rho[0] = e2;
             isq.v[0] = 1.0;
             const double stop = std::max(target, inner_rtol * beta);
             int nj = 0;
@@ -1904,30 +1911,32 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
                 if (s.cycles >= opts->max_cycles) { rc = STZMG_ERR_NOT_CONVERGED; break; }
                 float *w = h->kV32 + (long)(j + 1) * n3;
                 float *zj = h->kZ + (long)j * n3;
-                // z_j = M^-1 u_j, u_j in r32
+                // z_j = M^-1 2^e_j u_j, 2^e_j u_j in r32
                 if (!fine_zero_start(h))
                     hipLaunchKernelGGL((k_fill<float>), dim3(nblk(n3)), dim3(kThreads), 0, h->stream, L.x32, 0.0f, n3);
                 if ((rc = run_vcycles<float>(h, inner, graph, true))) return rc;
                 s.cycles += inner;
-                // w' = A z_j in FP32 (A M^-1 v_j is w' / nrm_j); the same
+                // w' = A z_j in FP32 (A M^-1 v_j is w' / rho_j); the same
                 // pass keeps z_j (x32 is overwritten by the next V-cycles)
                 launch_apply<float>(h, L, (const float *)L.x32, w, zj);
                 // c_i = (w', u_i) / nrm_i^2; w' -= sum c_i u_i; |w'|^2
                 launch_mdot_n<1, float>(h->stream, (const float *)w, (const float *)h->kV32, j + 1, n3, h->kpart);
                 hipLaunchKernelGGL(k_reduce_cols, dim3(j + 1), dim3(kThreads), 0, h->stream,
                                    (const double *)h->kpart, kDotBlocks, j + 1, h->kdev, hcol, 1, isq);
+                e2 = pow2(sigma / rho[j]);
                 launch_maxpy_n<1, float>(h->stream, w, (const float *)h->kV32, (const double *)h->kdev, j + 1, n3,
-                                         h->kpart, L.r32);
+                                         h->kpart, L.r32, (float)e2);
                 hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(kThreads), 0, h->stream, (const double *)h->kpart,
                                    kDotBlocks, 1, (double *)nullptr, hcol + (j + 1), 0, KrylovVals{});
                 LAUNCHCHK(h);
                 HIPCHK(h, hipStreamSynchronize(h->stream));
                 std::copy(hcol, hcol + j + 2, hc.begin());
                 const double wn = std::sqrt(hc[j + 1]);
-                for (int i = 0; i <= j; i++) Hc(i, j) = hc[i] * nrm[i] / nrm[j];
-                Hc(j + 1, j) = wn / nrm[j];
+                for (int i = 0; i <= j; i++) Hc(i, j) = hc[i] * nrm[i] / rho[j];
+                Hc(j + 1, j) = wn / rho[j];
                 if (!std::isfinite(wn)) { rc = STZMG_ERR_NONFINITE; break; }
                 nrm[j + 1] = wn;
+                rho[j + 1] = e2 * wn;
                 isq.v[j + 1] = wn > 0 ? 1.0 / (wn * wn) : 0.0;
                 for (int i = 0; i < j; i++) {
                     const double a = Hc(i, j), b = Hc(i + 1, j);
@@ -1951,7 +1960,7 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
                 y[i] = t / Hc(i, i);
             }
             KrylovVals yv{};
-            for (int i = 0; i < nj; i++) yv.v[i] = y[i] / nrm[i];
+            for (int i = 0; i < nj; i++) yv.v[i] = y[i] / rho[i];
             hipLaunchKernelGGL(k_xupdate<float>, dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, L.x64, (const float *)h->kZ,
                                yv, nj, n3);
             LAUNCHCHK(h);
@@ -1988,7 +1997,7 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
         const unsigned nb3 = nblk(n3);
         while (rc == 0 && s.res > target && beta > 0) {
             hipLaunchKernelGGL((k_scale<double, double>), dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, h->kV,
-                               (const double *)L.t64, 1.0 / beta, n3, (double *)nullptr);
+                               (const double *)L.t64, 1.0 / beta, n3, (double *)nullptr, 1.0);
             std::fill(g.begin(), g.end(), 0.0);
             g[0] = beta;
             int nj = 0;
@@ -2020,7 +2029,7 @@ int stzmg_solve(stzmg_t h, const stzmg_solve_opts *opts, stzmg_solve_stats *st) 
                 if (!std::isfinite(wn)) { rc = STZMG_ERR_NONFINITE; break; }
                 if (wn > 0)
                     hipLaunchKernelGGL((k_scale<double, double>), dim3(nblk_ew(n3)), dim3(kThreads), 0, h->stream, w,
-                                       (const double *)w, 1.0 / wn, n3, (double *)nullptr);
+                                       (const double *)w, 1.0 / wn, n3, (double *)nullptr, 1.0);
                 for (int i = 0; i < j; i++) {
                     const double a = Hc(i, j), b = Hc(i + 1, j);
                     Hc(i, j) = cs[i] * a + sn[i] * b;
