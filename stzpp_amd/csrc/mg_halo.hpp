@@ -434,13 +434,13 @@ __global__ __launch_bounds__((halo_threads<TX, TY>())) __attribute__((amdgpu_wav
     }
 
     // ---- the coefficient tables into the scalar cache ----
-    const T *A0 = pk + (long)kA * march_stride(KEY);
-    const T *A1 = pk + (long)(odd ? k0 + 1 : k0) * march_stride(KEY);
+    const T *A0 = pk + (long)kA * kMarchStride<KEY>;
+    const T *A1 = pk + (long)(odd ? k0 + 1 : k0) * kMarchStride<KEY>;
     {
         // every wave touches its share of the lines of the three rows
         constexpr int step = 64 / (int)sizeof(T), lines = (march_stride(KEY) + step - 1) / step;
         const int kB = plane(k0 + (odd ? 2 : 0));
-        const T *R[3] = {halo_row(pk + (long)k0 * march_stride(KEY)), halo_row(pk + (long)kB * march_stride(KEY)),
+        const T *R[3] = {halo_row(pk + (long)k0 * kMarchStride<KEY>), halo_row(pk + (long)kB * kMarchStride<KEY>),
                          halo_row(A1)};
         T touch = 0;
 #pragma unroll

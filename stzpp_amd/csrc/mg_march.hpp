@@ -118,6 +118,11 @@ __host__ __device__ constexpr int march_count(int pat, int phase) {
     return n;
 }
 __host__ __device__ constexpr int march_stride(int pat) { return march_count(pat, 0) + march_count(pat, 1); }
+// The same as a constant: a call in a kernel is evaluated there, block by
+// block in scalar loops, for the patterns without centrosymmetry (it took the
+// one-launch sweep of a shear pattern at 32 x 32 x 33 from 10 to 29 us).
+template <int PAT>
+constexpr int kMarchStride = march_stride(PAT);
 // Source of packed entry j: 9 b + e for operator entries (b < 27), 243 + e
 // for the inverse block.
 __host__ __device__ constexpr int march_src(int pat, int j) {
@@ -486,7 +491,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(march_waves<
             fetch(xs, k + 2, n1, zs);
             fetch(xo, k + 3, n2, zo);
         }
-        const T *A = pk + (long)k * march_stride(PAT);
+        const T *A = pk + (long)k * kMarchStride<PAT>;
 
         // phase Z: planes k-1 and k+1.  The two points of a pair are
         // addressed from the first one's window index (the second sits a

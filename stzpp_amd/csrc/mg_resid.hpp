@@ -155,7 +155,7 @@ __global__ __launch_bounds__(NT) void k_resid_march(Dims d, const T *__restrict_
 #pragma unroll
                 for (int c = 0; c < 3; c++) rv[u][c] = at_bytes(r + base + c * d.N, po + u * rstep);
         }
-        const T *A = pk + (long)k * march_stride(PAT);
+        const T *A = pk + (long)k * kMarchStride<PAT>;
         T acc[R][3];
 #pragma unroll
         for (int u = 0; u < R; u++) acc[u][0] = acc[u][1] = acc[u][2] = 0;

@@ -55,7 +55,7 @@ __global__ __launch_bounds__(kRRThreads) void k_resid_restrict(Dims F, Dims C, c
     const int ez = wv / 2, t0 = (wv & 1) * 64 + lane, t = t0 < NP ? t0 : 0;
     const int ty = t / RX, tx = t - ty * RX;
     const int k = plane(2 * K - 1 + ez), kc = k < 0 ? 0 : k;
-    const T *A = pk + (long)kc * march_stride(KEY);
+    const T *A = pk + (long)kc * kMarchStride<KEY>;
     T rv[3];
     {
         const long q = mn * kc + wrap1(2 * I0 - 1 + tx, F.m) + (long)F.m * wrap1(2 * J0 - 1 + ty, F.n);

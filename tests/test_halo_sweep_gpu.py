@@ -159,3 +159,25 @@ def test_residual_and_restriction_in_one_launch(kind, m, n, o, pz):
     xc, rc = mg.fields(1)
     assert not xc.any()
     assert relerr(rc, orc.fields(1)[1]) < 1e-12
+
+
+@pytest.mark.parametrize("kind", ["shear", "trans", "full"])
+@pytest.mark.parametrize("timed", [0, 2])  # FP64 sweep, FP32 sweep
+def test_patterns_without_symmetry_cost_no_more_than_dense(kind, timed):
+    """A zero pattern only takes entries out of the dense stencil's sums, so
+    its sweep is no slower than the dense one, also where no two opposite
+    blocks are equal.  Half as much again is left for the clock; the fault this
+    guards against took 2.3 times as long."""
+    m, n, o = 32, 32, 33
+    us = {}
+    for k in ("plain", kind):
+        planes = planes_of(k, m, n, o, 0)
+        rng = np.random.default_rng(8)
+        planes = planes * (1 + 1e-3 * rng.uniform(-1, 1, planes.shape))
+        mg = MG.Multigrid(m, n, o, (1, 1, 0), coarsest_total=m * n * o)
+        mg.setup_matrices_planes(planes)
+        mg.setup_fields(O.det_field(m * n * o, 81), O.det_field(m * n * o, 82))
+        mg.time_kernel(timed, 0, 50)
+        us[k] = 1e3 * min(mg.time_kernel(timed, 0, 50) for _ in range(5))
+    print(us, flush=True)
+    assert us[kind] < 1.5 * us["plain"]
