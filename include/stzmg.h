@@ -188,8 +188,10 @@ enum { STZMG_OPT_COARSE_KERNEL = 0, STZMG_OPT_FUSED_SMOOTHER = 1, STZMG_OPT_TILE
 /*   STZMG_OPT_FUSED_SMOOTHER 1 (default): per-plane levels with periodic x, y
  *                            (x and y sizes even and at least 8, more than
  *                            1024 points) sweep with two fused launches (one
- *                            per z parity) or, where small or not in tiles of
- *                            8, with one; 0: eight colour launches per sweep.
+ *                            per z parity) or, where small, with one; sides
+ *                            that are not multiples of 8 with one up to a few
+ *                            hundred thousand points and with eight colour
+ *                            launches beyond; 0: always eight.
  *   STZMG_OPT_TILED_RESIDUAL 1 (default): on the same levels the residual
  *                            marches tiles through z with planes staged in
  *                            LDS; 0: one thread per point reading its 27

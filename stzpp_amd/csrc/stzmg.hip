@@ -429,17 +429,32 @@ float *&xref_of<float>(Level &L) { return L.x32; }
 // launch (us per sweep, marching against one launch: 48 x 40 x 25, 390
 // workgroups, dense FP64 19.8 / 15.8, FP32 16.7 / 13.4; 48 x 48 x 24, 432,
 // shear FP64 14.4 / 13.1; 48 x 48 x 49, 900, FP64 15.0 / 21.0, FP32
-// 11.8 / 14.5; 64 x 64 x 33, 1088, FP64 18.4 / 30.5).  It also takes every
-// level that no marching tile divides, whose alternative is eight colour
-// launches (24 x 20 x 13 FP64 51 / 11.0).
+// 11.8 / 14.5; 64 x 64 x 33, 1088, FP64 18.4 / 30.5).
 constexpr long kHaloGroups = 512;
 
-// Fused-smoother tile class of a level for sweeps in type T: 0 none, 1 the
+// On a level that no marching tile divides the alternative is eight colour
+// launches, so there it goes further, until its arithmetic costs more than
+// their latency; the line depends on the zero pattern (index PAT_*: dense, no
+// corners, transformed, shear).  us per sweep, colours against one launch,
+// FP64 / FP32, centrosymmetric but for dense:
+//   dense         2304 workgroups 66 / 61 against 59 / 47, 2541 68 / 62 against
+//                 71 / 56, 4225 92 / 65 against 109 / 86
+//   no corners    3549 77 / 64 against 72 / 56, 4225 89 / 66 against 85 / 66
+//                 (8 % more without symmetry)
+//   transformed   4225 88 / 66 against 79 / 60, 4900 97 / 74 against 91 / 68
+//   shear         4225 88 / 66 against 76 / 59, 4900 96 / 74 against 85 / 66,
+//                 8450 115 / 92 against 144 / 111
+// (24 x 20 x 13, 78 workgroups, dense 51 / 50 against 9.9 / 9.1).
+constexpr long kHaloLone[4] = {2400, 3600, 4800, 4800};
+constexpr int kHaloWidest = PAT_SHEAR;  // the pattern whose line is the highest
+
+// Fused-smoother tile class of a level whose operator has zero pattern pat, for
+// sweeps in type T: 0 none, 1 the
 // large marching tiles of T (64 x 16 FP32, 32 x 16 FP64), 2 the 16 x 16
 // tiles, 3 the 8 x 8 tiles (the largest that divides the plane), 4 the
 // one-launch sweep.
 template <typename T>
-int fused_tile(const Level &L) {
+int fused_tile(const Level &L, int pat) {
     const Dims &d = L.d;
     if (!(L.mode == STZMG_OP_PLANE && d.px && d.py && d.o >= 4 && d.N > 1024)) return 0;
     int best = 0;
@@ -448,7 +463,7 @@ int fused_tile(const Level &L) {
     else if (d.m % kTinyTile == 0 && d.n % kTinyTile == 0) best = 3;
     const bool halo = STZ_MARCH != 0 && d.m % 2 == 0 && d.n % 2 == 0 && d.m >= 8 && d.n >= 8 && (!d.pz || d.o % 2 == 0);
     const long groups = (long)((d.m + kHaloTile - 1) / kHaloTile) * ((d.n + kHaloTile - 1) / kHaloTile) * ((d.o + 1) / 2);
-    if (halo && (best == 0 || groups <= kHaloGroups)) return 4;
+    if (halo && groups <= (best == 0 ? kHaloLone[pat] : kHaloGroups)) return 4;
     return best;
 }
 
@@ -1139,8 +1154,8 @@ int build_hierarchy_ops(stzmg_t h) {
         L.pat = pat;
         // centrosymmetric: block(-o) equal to block(o) in every plane
         L.sym = used[27] != 0;
-        L.ftile = fused_tile<float>(L);
-        L.ftile64 = fused_tile<double>(L);
+        L.ftile = fused_tile<float>(L, pat);
+        L.ftile64 = fused_tile<double>(L, pat);
         L.fused = h->fused_smoother && L.ftile && L.ftile64 && L.x64b;
         L.tiled = h->tiled_resid && tiled_ok(L);
         L.tiled_small = h->tiled_resid && tiled_small_ok(L);
@@ -1285,7 +1300,9 @@ int stzmg_create(const stzmg_desc *d, stzmg_t *out) {
             alloc(&L.inv32, L.ncls * 9) || alloc(&L.x64, n3) || alloc(&L.r64, n3) || alloc(&L.t64, n3) ||
             alloc(&L.x32, n3) || alloc(&L.r32, n3) || alloc(&L.t32, n3))
             return bail(fail(h, STZMG_ERR_NOMEM, "device allocation failed at level %zu", l));
-        if (fused_tile<float>(L) && fused_tile<double>(L) && (alloc(&L.x64b, n3) || alloc(&L.x32b, n3)))
+        // the second x of fused sweeps, wherever an operator may allow them
+        if (fused_tile<float>(L, kHaloWidest) && fused_tile<double>(L, kHaloWidest) &&
+            (alloc(&L.x64b, n3) || alloc(&L.x32b, n3)))
             return bail(fail(h, STZMG_ERR_NOMEM, "device allocation failed at level %zu", l));
         hipMemsetAsync(L.ops64, 0, sizeof(double) * L.ncls * kBlk, h->stream);
         hipMemsetAsync(L.x64, 0, sizeof(double) * n3, h->stream);

@@ -181,3 +181,29 @@ def test_patterns_without_symmetry_cost_no_more_than_dense(kind, timed):
         us[k] = 1e3 * min(mg.time_kernel(timed, 0, 50) for _ in range(5))
     print(us, flush=True)
     assert us[kind] < 1.5 * us["plain"]
+
+
+@pytest.mark.parametrize("kind,o,fused", [("plain", 47, True), ("plain", 49, False), ("full", 71, True),
+                                          ("full", 73, False), ("trans", 95, True), ("trans", 97, False),
+                                          ("shear", 95, True), ("shear", 97, False), ("plain", 161, False)])
+def test_large_level_that_no_tile_divides(kind, o, fused):
+    """76 x 76 points, 100 workgroups a plane pair: up to 2400 (dense), 3600 (no
+    corners) and 4800 (transformed, shear) workgroups sweep in one launch, more
+    in eight colour launches, which beat it there (100 x 100 x 100 dense 115 us
+    against 210).  Both compute the same sweep (rounding as above)."""
+    N = 76 * 76 * o
+    mg = MG.Multigrid(76, 76, o, (1, 1, 0), coarsest_total=N)
+    mg.setup_matrices_planes(planes_of(kind, 76, 76, o, 0))
+    x, r = O.det_field(N, 91), O.det_field(N, 92)
+    mg.setup_fields(x, r)
+    mg.gauss_seidel(0, 1)
+    got = mg.x(0)
+    if fused:
+        assert mg.time_kernel(4, 0, 1) > 0  # one launch of the fused sweep
+    else:
+        with pytest.raises(MG.MultigridError):
+            mg.time_kernel(4, 0, 1)
+    mg.set_option(MG.OPT_FUSED_SMOOTHER, 0)
+    mg.setup_fields(x, r)
+    mg.gauss_seidel(0, 1)
+    assert relerr(got, mg.x(0)) < 1e-12
