@@ -22,7 +22,7 @@
 #include <atomic>
 #include <cstddef>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 namespace stz {
@@ -125,7 +125,7 @@ class HostRing {
                     if (e != hipSuccess) err.store((int)e);
                     work(s);
                 });
-            } catch (const std::system_error &) {
+            } catch (const std::exception &) {  // no thread, or no memory for one
                 mine[s] = true;
             }
         }
