@@ -1,11 +1,14 @@
-"""The 16-lane colour pass of per-point operators (k_gs_points) and the
-register-resident bottom sweeps against the oracle.
+"""The 16-lane colour pass of per-point operators (k_gs_points) and the sweeps
+of the coarsest level, in the V-cycle and tabulated as x = Q r, against the
+oracle.
 
 Points: every kind of boundary (walls all around, periodic, an odd periodic
 size with its third colour), sizes whose colour passes end inside a row of
-lanes and inside a workgroup, and the smallest grid.  Bottom sweeps: the
-widest level they take (64 points of a colour), ones just beyond, odd planes
-between walls.  FP64 rounding of a 27-block sum stays far below 1e-12 of the
+lanes and inside a workgroup, and the smallest grid.  Bottom sweeps: without
+the map they run from the tables in the V-cycle; the map's form with tables and
+indices in registers takes levels of up to 64 points of a colour (16 x 16 x 16,
+16 x 16 x 8, 16 x 16 x 15, 20 x 12 x 9 and 12 x 20 x 12 here, the first and
+third at 64), its other form the rest (80, 72 and 96 points).  FP64 rounding of a 27-block sum stays far below 1e-12 of the
 largest value over a few sweeps, FP32 below 2e-6 in one.
 """
 import numpy as np
@@ -58,18 +61,20 @@ def test_point_sweep(m, n, o, prd):
     assert relerr(mg.x(0), orc.fields(0)[0]) < 2e-6
 
 
-@pytest.mark.parametrize("m,n,o,pz", [(16, 16, 16, 1), (16, 16, 8, 1), (16, 16, 17, 0), (20, 12, 9, 0), (24, 16, 9, 0),
-                                      (12, 20, 12, 1), (32, 16, 12, 1)])
+@pytest.mark.parametrize("m,n,o,pz", [(16, 16, 16, 1), (16, 16, 8, 1), (16, 16, 15, 0), (16, 16, 17, 0), (20, 12, 9, 0),
+                                      (24, 16, 9, 0), (12, 20, 12, 1), (32, 16, 12, 1)])
 @pytest.mark.parametrize("fp32", [False, True])
-def test_bottom_sweeps(m, n, o, pz, fp32):
+@pytest.mark.parametrize("bottom_map", [0, 1])
+def test_bottom_sweeps(m, n, o, pz, fp32, bottom_map):
     """Two-level V-cycles whose coarsest level runs its 24 sweeps in one
-    workgroup, against the oracle's."""
+    workgroup, at every cycle or once for each column of the map, against the
+    oracle's."""
     prd = (1, 1, pz)
     T = np.array([[1.05, 0.0, 0.2], [0.0, 1.0, 0.0], [0.0, 0.0, 0.95]])
     st = MG.trans_stencil(T, 1.0, 1.5, 1.0 / m, 1.0 / n, 1.0 / o, 1.0)
     fix = MG.shear_stencil(1.0, 1.5, 1.0 / m, 1.0 / n, 1.0 / o, 1.0)[1]
     mg = MG.Multigrid(m, n, o, prd)
-    mg.set_option(MG.OPT_BOTTOM_MAP, 0)
+    mg.set_option(MG.OPT_BOTTOM_MAP, bottom_map)
     mg.setup_matrices_const(st, None if pz else fix)
     assert mg.nlevels == 2
     orc = O.OracleMG(m, n, o, prd, mode=O.PLANE)
