@@ -1,12 +1,14 @@
 // Copies between device memory and a caller's pageable host memory.
 //
 // The runtime's own pageable copy moves such a transfer through one thread,
-// which also takes the first touch of every one of the caller's fresh pages.  Here up to kSlots worker threads each take every
-// kSlots-th chunk through a pinned slot of their own, so the transfers over
-// the bus, the memory copies and the page faults of different chunks overlap.
-// Measured (MI355X host, 8 threads): 311 MB state to the host 31.5 -> 9.8 ms,
-// a 14 MB cube 1.7 -> 0.67 ms (with one host copy less), 283 MB state to the
-// device 10.2 -> 7.6 ms.  Smaller transfers stay on the runtime's path, where
+// which also takes the first touch of every one of the caller's fresh pages.
+// Here up to kSlots worker threads each take every kSlots-th chunk through a
+// pinned slot of their own, so the transfers over the bus, the memory copies
+// and the page faults of different chunks overlap.  Output cubes and the
+// reference map take it; the state's fields do not.
+// Measured (MI355X host, 8 threads): a 14 MB cube to the host 1.7 -> 0.67 ms
+// (with one host copy less); fields of 311 MB in all to the host 31.5 -> 9.8 ms
+// and of 283 MB to the device 10.2 -> 7.6 ms.  Smaller transfers stay on the runtime's path, where
 // starting threads costs more than it gains: 64^3 cells (6 and 13 MB fields)
 // took 2.2 ms in threads against 2.05 ms, and uploads of 9 and 18 MB 1.0 ms
 // against 0.86 ms.

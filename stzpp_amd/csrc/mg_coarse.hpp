@@ -140,8 +140,9 @@ __device__ void wg_bottom_sweeps_reg(const Dims &d, const T *ops, const T *inv, 
     const int g = grp < tot ? grp : 0;
     const int ii = g % cntx, rest = g / cntx, jj = rest % cnty, kk = rest / cnty;
     // blocks h = 0, 1 of this lane, by plane parity; index parts of the
-    // neighbour by colour.  A block that does not exist (the centre, beyond
-    // the list, across a wall) is zero and reads the point itself.
+    // neighbour by colour.  A block that does not exist is zero: the centre and
+    // those beyond the list read the point itself, one across a wall a point of
+    // this plane.
     T A[2][2][9], B[2][3];
     int qx[2][2], qy[2][2], qz[2][2], pz[2];
     bool own[2];

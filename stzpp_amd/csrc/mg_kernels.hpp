@@ -170,8 +170,9 @@ __device__ __forceinline__ void gs_point(const Dims &d, T *__restrict__ x, const
 
 // One colour pass of block Gauss-Seidel over the points of colour
 // (cx,cy,cz).  Points of one colour are never stencil neighbours, so the pass
-// is order-independent.  Grid: (ceil(cntx*cnty/256), cntz).
-template <typename T, int MODE>
+// is order-independent.  Per-plane operators (per-point ones: k_gs_points).
+// Grid: (ceil(cntx*cnty/256), cntz).
+template <typename T>
 __global__ __launch_bounds__(kThreads) void k_gs(Dims d, T *__restrict__ x,
                                                  const T *__restrict__ r,
                                                  const T *__restrict__ ops,
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(kThreads) void k_gs(Dims d, T *__restrict__ x,
     const long t = (long)blockIdx.x * kThreads + threadIdx.x;
     if (t >= (long)cntx * cnty) return;
     const int jj = (int)(t / cntx), ii = (int)(t - (long)jj * cntx);
-    gs_point<T, MODE>(d, x, r, ops, inv, col_coord(ii, cx, d.m), col_coord(jj, cy, d.n), k);
+    gs_point<T, 0>(d, x, r, ops, inv, col_coord(ii, cx, d.m), col_coord(jj, cy, d.n), k);
 }
 
 // 1-D restriction weight of fine vertex 2I+e for coarse vertex I (vertex

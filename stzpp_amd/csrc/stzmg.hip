@@ -600,10 +600,12 @@ void launch_fused_pat(stzmg_t h, Level &L, bool zero_start, const Level *corr) {
 template <typename T>
 void launch_gs_sweep_colours(stzmg_t h, Level &L);
 
-// Whether a sweep of level L can start from x = 0 without the zeros in
-// memory (the fused sweep k_gs_march skips the planes it knows are zero).
+// Whether a sweep of level L can add the coarse level's correction itself
+// (k_gs_halo, as its window arrives).
 template <typename T>
 bool correction_ok(const Level &L) { return L.fused && (sizeof(T) == 4 ? L.ftile : L.ftile64) == 4; }
+// Whether it can start from x = 0 without the zeros in memory (k_gs_march
+// skips the planes it knows are zero, k_gs_halo reads none of x).
 bool zero_start_ok(const Level &L) { return STZ_MARCH != 0 && L.fused; }
 
 // One Gauss-Seidel sweep of a level: one or two fused launches where the
@@ -654,7 +656,7 @@ void launch_gs_sweep_colours(stzmg_t h, Level &L) {
                     continue;
                 }
                 dim3 g(nblk((long)cntx * cnty), cntz);
-                hipLaunchKernelGGL((k_gs<T, 0>), g, dim3(kThreads), 0, h->stream, d, x_of<T>(L),
+                hipLaunchKernelGGL((k_gs<T>), g, dim3(kThreads), 0, h->stream, d, x_of<T>(L),
                                    (const T *)r_of<T>(L), ops_of<T>(L), inv_of<T>(L), cx, cy, cz, cntx, cnty);
             }
 }
@@ -2122,7 +2124,7 @@ int stzmg_time_kernel(stzmg_t h, int kind, int level, int reps, double *ms_per_u
         ms /= reps;
     } else {
         // one event pair around each launch of the fused sweep (two per
-        // sweep): the mean kernel duration, without the gaps between launches
+        // sweep, one where the level sweeps in one launch): the mean kernel duration, without the gaps between launches
         std::vector<hipEvent_t> ev(4 * (size_t)reps);
         hipError_t e = hipSuccess;
         size_t made = 0;
