@@ -243,8 +243,11 @@ bool tiled_small_ok(const Level &L) {
 // 6 us a V-cycle and level (one V-cycle FP64 / FP32, two launches against
 // one: 32 x 32 x 33 150 / 133 -> 137 / 121 us; 64 x 64 x 65 with its 266,240
 // points 292 / 251 -> 280 / 240; 96 x 80 x 49, 376,320, 360 / 308 -> 334 /
-// 284); at 128 x 128 x 65 (1,064,960) the residuals computed twice cost more
-// than the launch (558 / 445 -> 571 / 457).
+// 284; 64 x 64 x 97, 397,312, 362 / 298 -> 353 / 289).  Above, the residuals
+// computed twice cost what the launch did or more: with it on the fine level
+// too 128 x 96 x 33, 405,504, 347 / 291 -> 350 / 292; 96 x 96 x 49, 451,584,
+// 381 / 321 -> 379 / 319; 128 x 64 x 65, 532,480, 516 / 417 -> 523 / 422;
+// 128 x 128 x 65, 1,064,960, 558 / 445 -> 571 / 457.
 constexpr long kRRMaxPoints = 400000;
 bool rr_ok(const Level &L) {
     return L.mode == STZMG_OP_PLANE && L.d.px && L.d.py && L.d.m % 2 == 0 && L.d.n % 2 == 0 && L.d.m >= 8 &&
