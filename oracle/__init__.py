@@ -1,7 +1,7 @@
 """CPU oracle for the STZ++ hot path -- TEST INFRASTRUCTURE ONLY.
 
 Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg import
-this package, and only as the checker.  It holds:
+this package, and only as what results are compared with.  It holds:
 
 * ``liboracle.so`` (mg_oracle.c): a plain-C FP64 restatement of the reference
   multigrid (mg_3d_template/region.cc, multigrid.cc) -- residual, lexicographic

@@ -3,7 +3,7 @@
  * This is a plain-C FP64 restatement of the reference's geometric multigrid
  * (mg_3d_template/region.cc, multigrid.cc) on one subdomain.  It is used by
  * tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg as the
- * checker; the product path never links or calls it.
+ * comparison; the product path never links or calls it.
  *
  * Conventions shared with the GPU library (include/stzmg.h):
  *   point index     p = i + m*(j + n*k)           (x fastest)
